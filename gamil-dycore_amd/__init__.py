@@ -455,12 +455,12 @@ class Dycore:
         self._ghs[member] = ghs.copy()
 
     def get_state(self, member=0):
-        u = np.zeros((self.M, self.N)); v = np.zeros((self.M - 1, self.N)); gd = np.zeros((self.M, self.N))
+        u = np.empty((self.M, self.N)); v = np.empty((self.M - 1, self.N)); gd = np.empty((self.M, self.N))
         _check(lib().gd_get_state(self.h, member, _dp(u), _dp(v), _dp(gd), self.N), self.h)
         return u, v, gd
 
     def diag_fields(self, member=0):
-        div = np.zeros((self.M, self.N)); vor = np.zeros((self.M - 1, self.N))
+        div = np.empty((self.M, self.N)); vor = np.empty((self.M - 1, self.N))
         _check(lib().gd_get_diag_fields(self.h, member, _dp(div), _dp(vor), self.N), self.h)
         return div, vor
 
@@ -491,7 +491,7 @@ class Dycore:
 
     # -- operator seams ----------------------------------------------------
     def space_operators(self, pass_="all", member=0):
-        du = np.zeros((self.M, self.N)); dv = np.zeros((self.M - 1, self.N)); dgd = np.zeros((self.M, self.N))
+        du = np.empty((self.M, self.N)); dv = np.empty((self.M - 1, self.N)); dgd = np.empty((self.M, self.N))
         _check(lib().gd_space_operators(self.h, member, PASS[pass_], _dp(du), _dp(dv), _dp(dgd), self.N), self.h)
         return du, dv, dgd
 

@@ -37,6 +37,16 @@ hipError_t launch_divvor(const Args &a, hipStream_t s);
 // check_antisymmetry's ten inner products (and their magnitudes) of member
 // a.m0's state X, left in its Tb dv field (entries 0..19; Tb du is scratch)
 hipError_t launch_terms(const Args &a, hipStream_t s);
+// k_rows: up to kRowBlocks blocks of rows between device rows (dpitch doubles
+// apart) and dense rows in pinned host memory
+constexpr int kRowBlocks = 4;
+struct RowsArg {
+  int nblk;
+  double *dev[kRowBlocks], *pin[kRowBlocks];
+  int rows[kRowBlocks], n[kRowBlocks];
+  int64_t dpitch[kRowBlocks];
+};
+hipError_t launch_rows(const RowsArg &a, bool to_host, hipStream_t s);
 hipError_t configure_kernels(int max_lds);
 // polar filter of the staged rows + rescale + phase epilogue (gd_filter.hip)
 hipError_t launch_filter(const Args &a, int prec, hipStream_t s);
