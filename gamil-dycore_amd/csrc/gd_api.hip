@@ -96,6 +96,10 @@ struct gd_handle {
   std::map<int, int> tuned_fused, tuned_wpm;
   std::vector<int> prow[2];
   FiltRow *dprow[2] = {nullptr, nullptr};
+  // pinned staging of host <-> device field copies (move_rows), grown on
+  // demand up to kPinBytes
+  double *pin = nullptr;
+  size_t pin_bytes = 0;
 };
 
 namespace {
@@ -125,10 +129,6 @@ void *dalloc(gd_handle *h, size_t bytes, hipError_t &e) {
   h->allocs.push_back(p);
   h->bytes += (int64_t)bytes;
   return p;
-  // pinned staging of host <-> device field copies (move_rows), grown on
-  // demand up to kPinBytes
-  double *pin = nullptr;
-  size_t pin_bytes = 0;
 }
 
 Args base_args(const gd_handle *h) {
@@ -954,6 +954,7 @@ int gd_destroy(gd_handle *h) {
   if (h->stream) hipStreamSynchronize(h->stream);
   for (auto &kv : h->graphs) hipGraphExecDestroy(kv.second);
   for (void *p : h->allocs) hipFree(p);
+  if (h->pin) hipHostFree(h->pin);
   if (h->stream) hipStreamDestroy(h->stream);
   delete h;
   return GD_OK;
@@ -1059,7 +1060,6 @@ int gd_get_state(gd_handle *h, int32_t member, double *u, double *v, double *gdp
   return move_rows(h, blk, n, true);
 }
 
-  if (h->pin) hipHostFree(h->pin);
 int gd_get_diag_fields(gd_handle *h, int32_t member, double *div, double *vor, int64_t ld) {
   int rc = check_member(h, member);
   if (rc) return rc;

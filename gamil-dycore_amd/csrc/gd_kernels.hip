@@ -536,24 +536,6 @@ __global__ void __launch_bounds__(64) k_terms_sum(const Args a) {
 }
 
 // ---------------------------------------------------------------------------
-// launchers
-// ---------------------------------------------------------------------------
-
-static inline int row_grid(int ntiles) { return ((ntiles + kXcd - 1) / kXcd) * kXcd; }
-
-template <typename CT>
-static hipError_t launch_tend_t(const Args &a, int pass, bool in_full, hipStream_t s) {
-  dim3 g(row_grid(a.ntiles)), b(kBlock);
-  const size_t lds = tend_lds_bytes(a, sizeof(CT));
-#define GD_TEND(P, F) hipLaunchKernelGGL((k_tend<CT, P, F>), g, b, lds, s, a)
-  if (pass == 0) { if (in_full) GD_TEND(0, true); else GD_TEND(0, false); }
-  else if (pass == 1) { if (in_full) GD_TEND(1, true); else GD_TEND(1, false); }
-  else { if (in_full) GD_TEND(2, true); else GD_TEND(2, false); }
-#undef GD_TEND
-  return hipGetLastError();
-}
-
-// ---------------------------------------------------------------------------
 // host <-> device copies of pitched rows through pinned memory
 // ---------------------------------------------------------------------------
 
@@ -581,6 +563,24 @@ hipError_t launch_rows(const RowsArg &a, bool to_host, hipStream_t s) {
     hipLaunchKernelGGL(k_rows<true>, g, b, 0, s, a);
   else
     hipLaunchKernelGGL(k_rows<false>, g, b, 0, s, a);
+  return hipGetLastError();
+}
+
+// ---------------------------------------------------------------------------
+// launchers
+// ---------------------------------------------------------------------------
+
+static inline int row_grid(int ntiles) { return ((ntiles + kXcd - 1) / kXcd) * kXcd; }
+
+template <typename CT>
+static hipError_t launch_tend_t(const Args &a, int pass, bool in_full, hipStream_t s) {
+  dim3 g(row_grid(a.ntiles)), b(kBlock);
+  const size_t lds = tend_lds_bytes(a, sizeof(CT));
+#define GD_TEND(P, F) hipLaunchKernelGGL((k_tend<CT, P, F>), g, b, lds, s, a)
+  if (pass == 0) { if (in_full) GD_TEND(0, true); else GD_TEND(0, false); }
+  else if (pass == 1) { if (in_full) GD_TEND(1, true); else GD_TEND(1, false); }
+  else { if (in_full) GD_TEND(2, true); else GD_TEND(2, false); }
+#undef GD_TEND
   return hipGetLastError();
 }
 
