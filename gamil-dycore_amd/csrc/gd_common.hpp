@@ -27,12 +27,70 @@ __device__ __forceinline__ int xcd_tile(int ntiles) {
 // kBlock); in every other launch the workgroup is one tile.
 __device__ __forceinline__ int ltid() { return (int)(threadIdx.x & (kBlock - 1)); }
 
+// x of another lane by a DPP move (CTRL: the DPP control of the move; every
+// lane active).
+template <int CTRL>
+__device__ __forceinline__ float dpp_mov(float x) {
+  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), CTRL, 0xf, 0xf, true));
+}
+template <int CTRL>
+__device__ __forceinline__ double dpp_mov(double x) {
+  return __hiloint2double(__builtin_amdgcn_update_dpp(0, __double2hiint(x), CTRL, 0xf, 0xf, true),
+                          __builtin_amdgcn_update_dpp(0, __double2loint(x), CTRL, 0xf, 0xf, true));
+}
+
+// The wave butterfly l <-> l ^ 32, 16, 8, 4, 2, 1 without LDS.  fold32(a, b):
+// in the lower half a's sums over l, l ^ 32, in the upper half b's
+// (v_permlane32_swap exchanges a's upper half with b's lower); fold16
+// likewise by rows of 16 (even rows a's, odd rows b's).  fold_row adds over l
+// ^ 8, 4, 2, 1: a rotation within the row of 16 gives lane l ^ n's value, since
+// the sums before it repeat with period 2 n.
+__device__ __forceinline__ double fold32(double a, double b) {
+  const auto lo = __builtin_amdgcn_permlane32_swap(__double2loint(a), __double2loint(b), false, false);
+  const auto hi = __builtin_amdgcn_permlane32_swap(__double2hiint(a), __double2hiint(b), false, false);
+  return __hiloint2double((int)hi[0], (int)lo[0]) + __hiloint2double((int)hi[1], (int)lo[1]);
+}
+__device__ __forceinline__ double fold16(double a, double b) {
+  const auto lo = __builtin_amdgcn_permlane16_swap(__double2loint(a), __double2loint(b), false, false);
+  const auto hi = __builtin_amdgcn_permlane16_swap(__double2hiint(a), __double2hiint(b), false, false);
+  return __hiloint2double((int)hi[0], (int)lo[0]) + __hiloint2double((int)hi[1], (int)lo[1]);
+}
+__device__ __forceinline__ double fold_row(double v) {
+  v += dpp_mov<0x128>(v);  // row_ror:8
+  v += dpp_mov<0x124>(v);
+  v += dpp_mov<0x122>(v);
+  v += dpp_mov<0x121>(v);
+  return v;
+}
+
+// Sum over the 64 lanes of a wave, the same in every lane.
+__device__ __forceinline__ double wave_sum(double v) {
+  v = fold32(v, v);
+  v = fold16(v, v);
+  return fold_row(v);
+}
+
+// The sums of K values over the wave, left in dst[0..K-1] (LDS) by the lanes
+// that hold them; four values to a butterfly.
+template <int K>
+__device__ __forceinline__ void wave_sums_to(const double (&v)[K], double *dst) {
+  const int lane = threadIdx.x & 63;
+#pragma unroll
+  for (int q = 0; q < K; q += 4) {
+    const int q1 = q + 1 < K ? q + 1 : q, q2 = q + 2 < K ? q + 2 : q, q3 = q + 3 < K ? q + 3 : q1;
+    const double s = fold_row(fold16(fold32(v[q], v[q1]), fold32(v[q2], v[q3])));
+    // lanes 0, 16, 32, 48 hold values q, q + 2, q + 1, q + 3
+    const int k = q + ((lane >> 4) & 1) * 2 + (lane >> 5);
+    if ((lane & 15) == 0 && k < K) dst[k] = s;
+  }
+}
+
 // Deterministic sum over the kBlock threads of a tile (fixed butterfly +
 // fixed cross-wave order); every thread of the tile returns the same value.
 // The barriers are the workgroup's, so every tile of a workgroup calls it
 // at the same point, each with its own `red`.
 __device__ __forceinline__ double block_sum(double v, double *red) {
-  for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
+  v = wave_sum(v);
   const int w = (threadIdx.x >> 6) & (kBlock / 64 - 1);
   __syncthreads();
   if ((threadIdx.x & 63) == 0) red[w] = v;
@@ -46,14 +104,9 @@ __device__ __forceinline__ double block_sum(double v, double *red) {
 // `red` holds 4*K doubles.  Every thread of the tile returns the same sums.
 template <int K>
 __device__ __forceinline__ void block_sum_n(double (&v)[K], double *red) {
-#pragma unroll
-  for (int q = 0; q < K; ++q)
-    for (int off = 32; off > 0; off >>= 1) v[q] += __shfl_xor(v[q], off, 64);
   const int w = (threadIdx.x >> 6) & (kBlock / 64 - 1);
   __syncthreads();
-  if ((threadIdx.x & 63) == 0)
-#pragma unroll
-    for (int q = 0; q < K; ++q) red[w * K + q] = v[q];
+  wave_sums_to<K>(v, red + w * K);
   __syncthreads();
 #pragma unroll
   for (int q = 0; q < K; ++q) {

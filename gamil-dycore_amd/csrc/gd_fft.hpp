@@ -480,14 +480,9 @@ __device__ __forceinline__ void filter_row(const Args &a, const Member &mb, cons
 // pass through the barriers, and every thread returns the sums.
 template <int K>
 __device__ __forceinline__ void head_sum_n(double (&v)[K], double *red) {
-#pragma unroll
-  for (int q = 0; q < K; ++q)
-    for (int off = 32; off > 0; off >>= 1) v[q] += __shfl_xor(v[q], off, 64);
   const int w = threadIdx.x >> 6;
   __syncthreads();
-  if ((threadIdx.x & 63) == 0 && w < kBlock / 64)
-#pragma unroll
-    for (int q = 0; q < K; ++q) red[w * K + q] = v[q];
+  if (w < kBlock / 64) wave_sums_to<K>(v, red + w * K);
   __syncthreads();
 #pragma unroll
   for (int q = 0; q < K; ++q) {
