@@ -26,6 +26,9 @@ namespace {
 
 thread_local std::string g_create_error;
 
+// Fewest rows worth strip tiles.
+constexpr int kStripMinRows = 8;
+
 // Staging rows of gd_filter_rows_noalloc: one array per device, resolved to
 // its device address once per device (g_scratch_ptr) when the first handle on
 // that device is created.  In host code the name `scratch` is only a host-side
@@ -34,6 +37,26 @@ constexpr size_t kScratchBytes = (size_t)4 << 20;
 static __device__ __align__(256) double scratch[kScratchBytes / sizeof(double)];
 std::mutex g_scratch_mu;
 std::map<int, double *> g_scratch_ptr;
+
+// Up to kMaxFarRng ranges of rows, as the row launches take them.
+struct RowRanges {
+  int n = 0, rows = 0;
+  int lo[kMaxFarRng] = {}, cnt[kMaxFarRng] = {};
+};
+
+// The rows of `list` (ascending) as ranges; false if they need too many.
+bool make_ranges(const std::vector<int> &list, RowRanges &r) {
+  r = RowRanges();
+  for (size_t k = 0; k < list.size(); ++k) {
+    if (k == 0 || list[k] != list[k - 1] + 1) {
+      if (r.n == kMaxFarRng) return false;
+      r.lo[r.n++] = list[k];
+    }
+    ++r.cnt[r.n - 1];
+    ++r.rows;
+  }
+  return true;
+}
 
 struct ProfEntry {
   std::string family;
@@ -69,15 +92,21 @@ struct gd_handle {
   std::vector<int> fft_rad;
   // fused phase launches (k_phase): the filter rows inside the tendency
   // launch; the row tiles cover the row ranges far_lo/far_cnt.  fused_ok:
-  // the shape allows them; wide_ok: also one workgroup per row (k_wphase);
+  // the shape allows them; wide_ok: also workgroups of two tiles (k_wphase);
   // fused_mode: -1 by launch size, 0 never, 1 always k_phase, 2 always
   // k_wphase where wide_ok
   bool fused_ok = false, wide_ok = false;
   int fused_mode = -1;
   int upd_narrow = -1;  // k_update rounds of four points and partials per thread: -1 by band size, 0 no, 1 yes
   int ncu = 256;  // compute units of the device
-  int nfar_rng = 0, nfar_rows = 0;
-  int far_lo[kMaxFarRng] = {}, far_cnt[kMaxFarRng] = {};
+  RowRanges far;        // rows with a component outside the filter, and the pole rows
+  // rows strip_a..strip_b (none: strip_b < strip_a) run as strip tiles in the
+  // phases of a fast or slow call; near_all is the rows around them, near_far
+  // those of them with a component outside the filter (and the pole rows)
+  int strip_a = 0, strip_b = -1;
+  RowRanges near_all, near_far;
+  void *dstrip = nullptr;
+  int strip_mode = -1;   // rows per strip tile: -1 by launch size
   int32_t *dstep = nullptr;
   double *ddiag = nullptr;  // [nmem][cap][3]
   int diag_cap = 512;
@@ -142,6 +171,9 @@ Args base_args(const gd_handle *h) {
   a.off_sx = h->off_sx;
   a.off_beta = h->off_beta;
   a.off_sy = h->off_sy;
+  a.strip_coef = h->dstrip;
+  a.nfar_rng = 1;
+  a.nfar_rows = a.far_cnt[0] = h->M;
   a.mslots = h->dmslots;
   a.mm_phi = h->dmm_phi;
   a.diag = h->ddiag;
@@ -225,18 +257,22 @@ hipError_t enqueue_filter(gd_handle *h, Args a) {
   return run(h, "filter", [&] { return launch_filter(a, h->prec, h->stream); });
 }
 
+void set_ranges(Args &a, const RowRanges &r, int nm) {
+  a.nfar_rng = r.n;
+  a.nfar_rows = r.rows;
+  for (int k = 0; k < kMaxFarRng; ++k) {
+    a.far_lo[k] = r.lo[k];
+    a.far_cnt[k] = r.cnt[k];
+  }
+  a.ntiles = nm * r.rows * a.nseg;
+}
+
 // The k_phase tiles of members 0..nm-1: their filter rows, then the row
-// tiles of the far-row ranges.
-void set_fused(const gd_handle *h, Args &a, int nm) {
+// tiles of the ranges.
+void set_fused(const gd_handle *h, Args &a, int nm, const RowRanges &r) {
   a.nnear = (int)(h->frows.size() / h->nmem) * nm;
   a.nnear_pad = ((a.nnear + kXcd - 1) / kXcd) * kXcd;
-  a.nfar_rng = h->nfar_rng;
-  a.nfar_rows = h->nfar_rows;
-  for (int k = 0; k < kMaxFarRng; ++k) {
-    a.far_lo[k] = h->far_lo[k];
-    a.far_cnt[k] = h->far_cnt[k];
-  }
-  a.ntiles = nm * h->nfar_rows * a.nseg;
+  set_ranges(a, r, nm);
 }
 
 // Fused phase launches pay off while a launch is a few rounds of resident
@@ -266,7 +302,7 @@ int phase_form(const gd_handle *h) {
   auto it = h->tuned_fused.find(h->nact);
   if (it != h->tuned_fused.end()) return it->second == 2 && !h->wide_ok ? 1 : it->second;
   if (h->wide_ok && (h->N + kSeg - 1) / kSeg == 2) {
-    const int64_t wgs = (int64_t)h->nact * ((int64_t)(h->frows.size() / h->nmem) + h->nfar_rows);
+    const int64_t wgs = (int64_t)h->nact * ((int64_t)(h->frows.size() / h->nmem) + h->far.rows);
     if (wgs <= 2 * (int64_t)h->ncu) return 2;
   }
   const int64_t tiles = (int64_t)h->nact * h->M * ((h->N + kSeg - 1) / kSeg);
@@ -275,17 +311,50 @@ int phase_form(const gd_handle *h) {
 
 bool use_fused(const gd_handle *h) { return phase_form(h) != 0; }
 
+// Rows per strip tile, 0 for none (GD_STRIP in the environment when the handle
+// is created forces a number).  A tile of R rows forms R + 2 rows; two rows
+// keep a small launch short, four repeat less.  Measured on MI355X, ms per step
+// with 2 / 4 / 8 rows: 720x361 0.355 / 0.375, four runs of 360x181 0.368 /
+// 0.326, 16 of them 0.782 / 0.734 / 0.787, 1440x721 0.757 / 0.727 / 0.775, 64 of
+// 360x181 3.90 / 3.69 / 3.64.
+int strip_rows(const gd_handle *h) {
+  if (h->strip_mode >= 0) return h->strip_mode;
+  const int64_t far = h->strip_b - h->strip_a + 1, nseg = (h->N + kSeg - 1) / kSeg;
+  return h->nact * nseg * ((far + 1) / 2) <= 2 * (int64_t)h->ncu ? 2 : 4;
+}
+
+// Form of the phase launches of a call with strip tiles, unless the handle's
+// form is forced or tuned: k_wphase (shortest chain of a filter row) while its
+// workgroups fit about two per CU, else k_phase.  Measured on MI355X, ms per
+// step: 360x181 0.241 against 0.267 (k_phase), four of them 0.326 / 0.341,
+// 720x361 0.355 / 0.366; 0.533 / 0.461 for two of 720x361.
+int strip_form(const gd_handle *h) {
+  if (!h->fused_ok || h->fused_mode >= 0 || h->tuned_fused.count(h->nact)) return phase_form(h);
+  const int64_t nact = h->nact, nseg = (h->N + kSeg - 1) / kSeg;
+  if (h->wide_ok) {
+    const int64_t R = strip_rows(h), groups = (h->strip_b - h->strip_a + R) / R;
+    const int64_t wgs = nact * (int64_t)(h->frows.size() / h->nmem) +
+                        (nact * nseg * (h->near_far.rows + groups) + 1) / 2;
+    if (10 * wgs <= 22 * (int64_t)h->ncu) return 2;
+  }
+  return 1;
+}
+
 // One tendency phase (a.phase) of the active members with its filter rows:
-// one k_phase launch, or k_tend then k_filter.
-hipError_t enqueue_phase(gd_handle *h, Args a, int pass, bool in_full) {
-  a.ntiles = h->nact * h->M * a.nseg;
-  const int form = phase_form(h);
+// one fused launch, or k_tend then k_filter.  strip: the rows strip_a..strip_b
+// run as strip tiles.
+hipError_t enqueue_phase(gd_handle *h, Args a, int pass, bool in_full, bool strip = false) {
+  const int form = strip ? strip_form(h) : phase_form(h);
   if (form == 0) {
+    if (strip)
+      set_ranges(a, h->near_all, h->nact);
+    else
+      a.ntiles = h->nact * h->M * a.nseg;
     hipError_t e = run(h, "tend", [&] { return launch_tend(a, h->prec, pass, in_full, h->stream); });
     if (e != hipSuccess) return e;
     return enqueue_filter(h, a);
   }
-  set_fused(h, a, h->nact);
+  set_fused(h, a, h->nact, strip ? h->near_far : h->far);
   if (form == 2) return run(h, "wphase", [&] { return launch_wphase(a, h->prec, pass, in_full, h->stream); });
   return run(h, "phase", [&] { return launch_phase(a, h->prec, pass, in_full, h->stream); });
 }
@@ -298,15 +367,24 @@ hipError_t enqueue_call(gd_handle *h, double dt, int pass, int s0, int s_out, in
   a.dt = dt;
   a.hdt = dt * 0.5;
   hipError_t e;
+  a.s0 = s0;
+  const bool strip = pass != GD_PASS_ALL && h->strip_b >= h->strip_a && strip_rows(h) > 0;
+  if (strip) {
+    a.strip_a = h->strip_a;
+    a.strip_b = h->strip_b;
+    a.strip_r = strip_rows(h);
+    a.strip_ngroup = (h->strip_b - h->strip_a + a.strip_r) / a.strip_r;
+    a.nstrip = h->nact * a.strip_ngroup * a.nseg;
+  }
   // first predictor: T = L(S0), S1 = S0 + dt/2 T
-  a.phase = PH_A; a.s_in = s0; a.s0 = s0; a.s_out = SP1;
-  if ((e = enqueue_phase(h, a, pass, s0 == SX)) != hipSuccess) return e;
+  a.phase = PH_A; a.s_in = s0; a.s_out = SP1;
+  if ((e = enqueue_phase(h, a, pass, s0 == SX, strip)) != hipSuccess) return e;
   // second predictor: T = L(S1), S2 = S0 + dt/2 T, keep T
   a.phase = PH_B; a.s_in = SP1; a.s_out = SP2;
-  if ((e = enqueue_phase(h, a, pass, false)) != hipSuccess) return e;
+  if ((e = enqueue_phase(h, a, pass, false, strip)) != hipSuccess) return e;
   // corrector tendency T = L(S2) and the beta inner-product partials
   a.phase = PH_C; a.s_in = SP2;
-  if ((e = enqueue_phase(h, a, pass, false)) != hipSuccess) return e;
+  if ((e = enqueue_phase(h, a, pass, false, strip)) != hipSuccess) return e;
   a.s_out = s_out;
   return run(h, "update", [&] { return launch_update(a, h->prec, h->stream); });
 }
@@ -331,7 +409,7 @@ hipError_t enqueue_diffusion(gd_handle *h, int s_in, bool in_full, double dt) {
     if (a.lap_final && use_fused(h)) {
       // the last application with its filter rows in one launch
       Args f = a;
-      set_fused(h, f, h->nact);
+      set_fused(h, f, h->nact, h->far);
       return run(h, "diffuse", [&] { return launch_dphase(f, h->prec, h->stream); });
     }
     e = run(h, "diffuse", [&] { return launch_diffuse(a, h->prec, h->stream); });
@@ -822,21 +900,34 @@ int gd_create(const gd_config *cfg, int32_t n_members, gd_handle **out) {
                       (j <= h->M - 2 && rc[j].stage[CDV] < 0);
       if (pole || un) far.push_back(j);
     }
-    int nr = 0;
-    bool fits = true;
-    for (size_t k = 0; k < far.size(); ++k) {
-      if (k == 0 || far[k] != far[k - 1] + 1) {
-        if (nr == kMaxFarRng) { fits = false; break; }
-        h->far_lo[nr] = far[k];
-        h->far_cnt[nr] = 0;
-        ++nr;
+    const bool fits = make_ranges(far, h->far);
+    // the strip tiles' rows: the longest run of rows with no component in the
+    // filter, no pole row and none next to one
+    int best = 0, end = -1;
+    for (int j = 2, run = 0; j <= h->M - 4; ++j) {
+      const bool clear = rc[j].stage[CDU] < 0 && rc[j].stage[CDV] < 0 && rc[j].stage[CDGD] < 0;
+      run = clear ? run + 1 : 0;
+      if (run > best) {
+        best = run;
+        end = j;
       }
-      ++h->far_cnt[nr - 1];
     }
-    h->nfar_rng = nr;
-    h->nfar_rows = (int)far.size();
+    const int ba = end - best + 1, bb = end;
+    if (fits && best >= kStripMinRows) {
+      std::vector<int> all, part;
+      for (int j = 0; j < h->M; ++j)
+        if (j < ba || j > bb) all.push_back(j);
+      for (int j : far)
+        if (j < ba || j > bb) part.push_back(j);
+      if (make_ranges(all, h->near_all) && make_ranges(part, h->near_far)) {
+        h->strip_a = ba;
+        h->strip_b = bb;
+      }
+    }
     const char *env = std::getenv("GD_FUSED");
     h->fused_mode = env && env[0] >= '0' && env[0] <= '2' ? env[0] - '0' : -1;
+    const char *bd = std::getenv("GD_STRIP");
+    if (bd && bd[0]) h->strip_mode = std::max(0, std::min(std::atoi(bd), 32));
     const char *nar = std::getenv("GD_UPD_NARROW");
     h->upd_narrow = nar && (nar[0] == '0' || nar[0] == '1') ? nar[0] - '0' : -1;
     // (the MFMA filter runs as its own launch between k_tend and k_filter)
@@ -907,7 +998,10 @@ int gd_create(const gd_config *cfg, int32_t n_members, gd_handle **out) {
       return fail(nullptr, GD_ERR_HIP, "device allocation failed");
     }
   }
-  if (!h->ddiag || !h->dcoef || !h->dslots || !h->dfrows || !h->dtwid ||
+  std::vector<unsigned char> strip_tab;
+  strip_rows_fill(rc, h->prec, strip_tab);
+  h->dstrip = dalloc(h, strip_tab.size(), e);
+  if (!h->dstrip || !h->ddiag || !h->dcoef || !h->dslots || !h->dfrows || !h->dtwid ||
       !h->dstep || !h->dghost || !h->dprow[0] || !h->dprow[1] || !h->dmslots) {
     gd_destroy(h);
     return fail(nullptr, GD_ERR_HIP, "device allocation failed");
@@ -922,6 +1016,7 @@ int gd_create(const gd_config *cfg, int32_t n_members, gd_handle **out) {
     tw[2 * k + 1] = (double)sinl(ang);
   }
   hipMemcpyAsync(h->dcoef, rc.data(), sizeof(RowCoef) * h->M, hipMemcpyHostToDevice, h->stream);
+  hipMemcpyAsync(h->dstrip, strip_tab.data(), strip_tab.size(), hipMemcpyHostToDevice, h->stream);
   if (nslots) hipMemcpyAsync(h->dslots, h->slots.data(), sizeof(StageSlot) * nslots, hipMemcpyHostToDevice, h->stream);
   if (!h->frows.empty())
     hipMemcpyAsync(h->dfrows, h->frows.data(), sizeof(FiltRow) * h->frows.size(), hipMemcpyHostToDevice, h->stream);
@@ -1417,7 +1512,7 @@ int gd_time_kernel(gd_handle *h, int32_t kernel, int32_t reps, double *us) {
     }
     if (kernel == GD_TIME_PHASE) {
       Args f = a;
-      set_fused(h, f, h->nmem);
+      set_fused(h, f, h->nmem, h->far);
       if (phase_form(h) == 2) return launch_wphase(f, h->prec, pass, false, h->stream);
       return launch_phase(f, h->prec, pass, false, h->stream);
     }

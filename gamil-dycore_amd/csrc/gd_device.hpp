@@ -128,10 +128,18 @@ struct Args {
   // k_phase: nnear whole-row filter tiles (one per FiltRow of the active
   // members; blocks 0..nnear_pad-1), then row tiles over the rows with a
   // component outside the filter, given as nfar_rng ranges of far_cnt[k]
-  // rows from far_lo[k] (nfar_rows rows in all)
+  // rows from far_lo[k] (nfar_rows rows in all).  k_tend: the rows of its
+  // tiles, in the same form.
   int nnear, nnear_pad;
   int nfar_rng, nfar_rows;
   int far_lo[kMaxFarRng], far_cnt[kMaxFarRng];
+  // strip tiles of the phase launches and k_tend: rows strip_a..strip_b in
+  // strip_ngroup groups of strip_r rows, nstrip tiles (member, group, segment) in
+  // strip_blk blocks after row_blk blocks of row tiles; coefficients strip_coef
+  // (strip_rows_fill)
+  int strip_a, strip_b, strip_r, strip_ngroup;
+  int nstrip, strip_blk, row_blk;
+  const void *strip_coef;
   int in_full;                 // k_diffuse: read stored u, v of s_in
   int nslots;
   int upd_wpm, nmem_launch;    // k_update: workgroups per member, members

@@ -20,6 +20,7 @@
 #include "gd_geom.hpp"
 #include "gd_common.hpp"
 #include "gd_launch.hpp"
+#include "gd_strip.hpp"
 #include "gd_tend.hpp"
 #include "gd_diffuse.hpp"
 
@@ -30,13 +31,21 @@ namespace gd {
 // ---------------------------------------------------------------------------
 
 // One tile per (member, row, segment), remapped so each XCD owns a
-// contiguous band of rows (tend_tile, gd_tend.hpp).
-template <typename CT, int PASS, bool IN_FULL>
+// contiguous band of rows (tend_tile, gd_tend.hpp); then the launch's strip
+// tiles.
+// (STRIP is apart because those tiles need more VGPRs.)
+template <typename CT, int PASS, bool IN_FULL, bool STRIP>
 __global__ void __launch_bounds__(kBlock) k_tend(const Args a) {
   extern __shared__ __align__(16) unsigned char smem[];
   __shared__ double red[4 * 6];
-  const int t = xcd_tile(a.ntiles);
-  if (t < 0) return;
+  if constexpr (STRIP) {
+    if ((int)blockIdx.x >= a.row_blk) {
+      strip_block<CT, PASS, IN_FULL>(a, a.row_blk, smem);
+      return;
+    }
+  }
+  const int b = blockIdx.x, t = (b % kXcd) * (a.row_blk / kXcd) + b / kXcd;
+  if (t >= a.ntiles) return;
   tend_tile<CT, PASS, IN_FULL, false>(a, t, smem, red);
 }
 
@@ -573,13 +582,20 @@ hipError_t launch_rows(const RowsArg &a, bool to_host, hipStream_t s) {
 static inline int row_grid(int ntiles) { return ((ntiles + kXcd - 1) / kXcd) * kXcd; }
 
 template <typename CT>
-static hipError_t launch_tend_t(const Args &a, int pass, bool in_full, hipStream_t s) {
-  dim3 g(row_grid(a.ntiles)), b(kBlock);
+static hipError_t launch_tend_t(Args a, int pass, bool in_full, hipStream_t s) {
+  a.row_blk = row_grid(a.ntiles);
+  a.strip_blk = strip_blocks(a, 1);
+  dim3 g(a.row_blk + a.strip_blk), b(kBlock);
   const size_t lds = tend_lds_bytes(a, sizeof(CT));
-#define GD_TEND(P, F) hipLaunchKernelGGL((k_tend<CT, P, F>), g, b, lds, s, a)
-  if (pass == 0) { if (in_full) GD_TEND(0, true); else GD_TEND(0, false); }
-  else if (pass == 1) { if (in_full) GD_TEND(1, true); else GD_TEND(1, false); }
-  else { if (in_full) GD_TEND(2, true); else GD_TEND(2, false); }
+#define GD_TEND(P, F, MR) hipLaunchKernelGGL((k_tend<CT, P, F, MR>), g, b, lds, s, a)
+  if (a.nstrip > 0) {
+    if (pass == 0) return hipErrorInvalidValue;
+    if (pass == 1) { if (in_full) GD_TEND(1, true, true); else GD_TEND(1, false, true); }
+    else { if (in_full) GD_TEND(2, true, true); else GD_TEND(2, false, true); }
+  }
+  else if (pass == 0) { if (in_full) GD_TEND(0, true, false); else GD_TEND(0, false, false); }
+  else if (pass == 1) { if (in_full) GD_TEND(1, true, false); else GD_TEND(1, false, false); }
+  else { if (in_full) GD_TEND(2, true, false); else GD_TEND(2, false, false); }
 #undef GD_TEND
   return hipGetLastError();
 }

@@ -12,6 +12,11 @@ namespace gd {
 
 __host__ __device__ inline size_t align16(size_t x) { return (x + 15) & ~(size_t)15; }
 
+// Blocks padded to a multiple of the XCDs, and the blocks of a launch's strip
+// tiles at `tiles` to a block.
+inline int pad_xcd(int n) { return (n + kXcd - 1) / kXcd * kXcd; }
+inline int strip_blocks(const Args &a, int tiles) { return a.nstrip > 0 ? pad_xcd((a.nstrip + tiles - 1) / tiles) : 0; }
+
 // k_filter: twiddle table (N complex) + two FFT buffers of L complex points.
 size_t filter_lds_bytes(int N, int L);
 
@@ -21,6 +26,8 @@ size_t tend_lds_bytes(const Args &a, size_t cts);
 
 // prec: 0 = FP64 plain, 1 = mixed (FP32 compute type)
 hipError_t launch_tend(const Args &a, int prec, int pass, bool in_full, hipStream_t s);
+// the coefficient rows of the strip tiles (gd_strip.hpp)
+void strip_rows_fill(const std::vector<RowCoef> &rc, int prec, std::vector<unsigned char> &out);
 // beta of predict_correct and the corrector update in one launch
 // (upd_wpm workgroups for each of nmem_launch members)
 hipError_t launch_update(const Args &a, int prec, hipStream_t s);

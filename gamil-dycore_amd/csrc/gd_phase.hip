@@ -20,6 +20,7 @@
 
 #include <cstdint>
 
+#include "gd_strip.hpp"
 #include "gd_common.hpp"
 #include "gd_device.hpp"
 #include "gd_fft.hpp"
@@ -122,14 +123,16 @@ __device__ __forceinline__ void near_tile(const Args &a, const FiltRow fr, unsig
 
 // Four longitudes per thread (rows up to 1024): five waves per SIMD (at most
 // 96 VGPRs); with the LDS of an FP64 tile that is five tiles per CU, so a
-// 720x361 run's phase fits in one round of resident workgroups.  Eight
-// (rows up to 2048): the twiddle table and row buffer of a 1440-point row
-// hold the LDS to three tiles per CU, so three waves per SIMD.
-template <int KP>
-constexpr int phase_waves() { return KP == 4 ? 5 : 3; }
+// 720x361 run's phase fits in one round of resident workgroups.  Beside strip
+// tiles a launch has far fewer workgroups, and four waves per SIMD (no spills)
+// are faster: 720x361 FP64 0.376 -> 0.350 ms per step.  Eight (rows up to
+// 2048): the twiddle table and row buffer of a 1440-point row hold the LDS to
+// three tiles per CU, so three waves per SIMD.
+template <int KP, bool STRIP>
+constexpr int phase_waves() { return KP == 4 ? (STRIP ? 4 : 5) : 3; }
 
-template <typename CT, int PASS, bool IN_FULL, int KP>
-__global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(phase_waves<KP>(), 8)))
+template <typename CT, int PASS, bool IN_FULL, int KP, bool STRIP>
+__global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(phase_waves<KP, STRIP>(), 8)))
 k_phase(const Args a) {
   extern __shared__ __align__(16) unsigned char smem[];
   __shared__ double red[4 * 6];
@@ -144,9 +147,15 @@ k_phase(const Args a) {
     if (t < a.nnear) near_tile<CT, PASS, IN_FULL, KP>(a, a.frows[t], smem, red);
     return;
   }
-  // row tiles: each XCD owns a contiguous band of them (nnear_pad and the
-  // remaining grid are multiples of kXcd, so block b stays on XCD b % kXcd)
-  const int bb = b - a.nnear_pad, per = (gridDim.x - a.nnear_pad) / kXcd;
+  if constexpr (STRIP) {
+    if (b >= a.nnear_pad + a.row_blk) {
+      strip_block<CT, PASS, IN_FULL>(a, a.nnear_pad + a.row_blk, smem);
+      return;
+    }
+  }
+  // row tiles: each XCD owns a contiguous band of them (nnear_pad and
+  // row_blk are multiples of kXcd, so block b stays on XCD b % kXcd)
+  const int bb = b - a.nnear_pad, per = a.row_blk / kXcd;
   const int t = (bb % kXcd) * per + bb / kXcd;
   if (t >= a.ntiles) return;
   tend_tile<CT, PASS, IN_FULL, true>(a, t, smem, red);
@@ -256,8 +265,9 @@ __device__ __forceinline__ void wnear_tile(const Args &a, const FiltRow fr, unsi
 
 // Two workgroups per CU (16 of the 20 waves that 96 VGPRs allow).  KW:
 // longitudes per thread in the filter (1 up to 512 longitudes, 2 up to 1024).
-template <typename CT, int PASS, bool IN_FULL, int KW>
-__global__ void __launch_bounds__(kWTiles * kBlock) __attribute__((amdgpu_waves_per_eu(5, 8)))
+// STRIP: with strip tiles (four waves per SIMD, as k_phase).
+template <typename CT, int PASS, bool IN_FULL, int KW, bool STRIP>
+__global__ void __launch_bounds__(kWTiles * kBlock) __attribute__((amdgpu_waves_per_eu(STRIP ? 4 : 5, 8)))
 k_wphase(const Args a) {
   extern __shared__ __align__(16) unsigned char smem[];
   __shared__ double red[kWTiles * 4 * 6];
@@ -267,8 +277,14 @@ k_wphase(const Args a) {
     if (t < a.nnear) wnear_tile<CT, PASS, IN_FULL, KW>(a, a.frows[t], smem, red);
     return;
   }
+  if constexpr (STRIP) {
+    if (b >= a.nnear_pad + a.row_blk) {
+      strip_block<CT, PASS, IN_FULL, kWTiles>(a, a.nnear_pad + a.row_blk, smem);
+      return;
+    }
+  }
   // row workgroups: tiles 2 r and 2 r + 1, each XCD owning a contiguous band
-  const int bb = b - a.nnear_pad, per = (gridDim.x - a.nnear_pad) / kXcd;
+  const int bb = b - a.nnear_pad, per = a.row_blk / kXcd;
   const int r = (bb % kXcd) * per + bb / kXcd;
   const int t0 = r * kWTiles;
   if (t0 >= a.ntiles) return;
@@ -341,7 +357,7 @@ __device__ __forceinline__ void dnear_tile(const Args &a, const FiltRow fr, unsi
 }
 
 template <typename CT, int KP>
-__global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(phase_waves<KP>(), 8)))
+__global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(phase_waves<KP, false>(), 8)))
 k_dphase(const Args a) {
   extern __shared__ __align__(16) unsigned char smem[];
   __shared__ double red[4 * 6];
@@ -380,14 +396,20 @@ size_t phase_lds_bytes(int N, int L, int prec) {
 }
 
 template <typename CT, int KP>
-static hipError_t launch_phase_k(const Args &a, int pass, bool in_full, hipStream_t s) {
-  const int rows = ((a.ntiles + kXcd - 1) / kXcd) * kXcd;
-  dim3 g(a.nnear_pad + rows), b(kBlock);
+static hipError_t launch_phase_k(Args a, int pass, bool in_full, hipStream_t s) {
+  a.row_blk = pad_xcd(a.ntiles);
+  a.strip_blk = strip_blocks(a, 1);
+  dim3 g(a.nnear_pad + a.row_blk + a.strip_blk), b(kBlock);
   const size_t lds = phase_lds_t<CT>(a.N, a.fft_L);
-#define GD_PH(P, F) hipLaunchKernelGGL((k_phase<CT, P, F, KP>), g, b, lds, s, a)
-  if (pass == 0) { if (in_full) GD_PH(0, true); else GD_PH(0, false); }
-  else if (pass == 1) { if (in_full) GD_PH(1, true); else GD_PH(1, false); }
-  else { if (in_full) GD_PH(2, true); else GD_PH(2, false); }
+#define GD_PH(P, F, S) hipLaunchKernelGGL((k_phase<CT, P, F, KP, S>), g, b, lds, s, a)
+  if (a.nstrip > 0) {
+    if (pass == 0) return hipErrorInvalidValue;
+    if (pass == 1) { if (in_full) GD_PH(1, true, true); else GD_PH(1, false, true); }
+    else { if (in_full) GD_PH(2, true, true); else GD_PH(2, false, true); }
+  }
+  else if (pass == 0) { if (in_full) GD_PH(0, true, false); else GD_PH(0, false, false); }
+  else if (pass == 1) { if (in_full) GD_PH(1, true, false); else GD_PH(1, false, false); }
+  else { if (in_full) GD_PH(2, true, false); else GD_PH(2, false, false); }
 #undef GD_PH
   return hipGetLastError();
 }
@@ -400,15 +422,20 @@ hipError_t launch_phase(const Args &a, int prec, int pass, bool in_full, hipStre
 }
 
 template <typename CT, int KW>
-static hipError_t launch_wphase_k(const Args &a, int pass, bool in_full, hipStream_t s) {
-  const int nwg = (a.ntiles + kWTiles - 1) / kWTiles;  // row workgroups
-  const int rows = ((nwg + kXcd - 1) / kXcd) * kXcd;
-  dim3 g(a.nnear_pad + rows), b(kWTiles * kBlock);
+static hipError_t launch_wphase_k(Args a, int pass, bool in_full, hipStream_t s) {
+  a.row_blk = pad_xcd((a.ntiles + kWTiles - 1) / kWTiles);  // row workgroups
+  a.strip_blk = strip_blocks(a, kWTiles);
+  dim3 g(a.nnear_pad + a.row_blk + a.strip_blk), b(kWTiles * kBlock);
   const size_t lds = wphase_lds<CT>(a.N, a.fft_L);
-#define GD_PH(P, F) hipLaunchKernelGGL((k_wphase<CT, P, F, KW>), g, b, lds, s, a)
-  if (pass == 0) { if (in_full) GD_PH(0, true); else GD_PH(0, false); }
-  else if (pass == 1) { if (in_full) GD_PH(1, true); else GD_PH(1, false); }
-  else { if (in_full) GD_PH(2, true); else GD_PH(2, false); }
+#define GD_PH(P, F, S) hipLaunchKernelGGL((k_wphase<CT, P, F, KW, S>), g, b, lds, s, a)
+  if (a.nstrip > 0) {
+    if (pass == 0) return hipErrorInvalidValue;
+    if (pass == 1) { if (in_full) GD_PH(1, true, true); else GD_PH(1, false, true); }
+    else { if (in_full) GD_PH(2, true, true); else GD_PH(2, false, true); }
+  }
+  else if (pass == 0) { if (in_full) GD_PH(0, true, false); else GD_PH(0, false, false); }
+  else if (pass == 1) { if (in_full) GD_PH(1, true, false); else GD_PH(1, false, false); }
+  else { if (in_full) GD_PH(2, true, false); else GD_PH(2, false, false); }
 #undef GD_PH
   return hipGetLastError();
 }
@@ -427,9 +454,11 @@ size_t wphase_lds_bytes(int N, int L, int prec) {
 
 template <typename CT, int KW>
 static hipError_t configure_wphase_k(int max_lds) {
-  const void *fns[] = {(const void *)k_wphase<CT, 0, true, KW>,  (const void *)k_wphase<CT, 0, false, KW>,
-                       (const void *)k_wphase<CT, 1, true, KW>,  (const void *)k_wphase<CT, 1, false, KW>,
-                       (const void *)k_wphase<CT, 2, true, KW>,  (const void *)k_wphase<CT, 2, false, KW>};
+  const void *fns[] = {(const void *)k_wphase<CT, 0, true, KW, false>, (const void *)k_wphase<CT, 0, false, KW, false>,
+                       (const void *)k_wphase<CT, 1, true, KW, false>, (const void *)k_wphase<CT, 1, false, KW, false>,
+                       (const void *)k_wphase<CT, 2, true, KW, false>, (const void *)k_wphase<CT, 2, false, KW, false>,
+                       (const void *)k_wphase<CT, 1, true, KW, true>,  (const void *)k_wphase<CT, 1, false, KW, true>,
+                       (const void *)k_wphase<CT, 2, true, KW, true>,  (const void *)k_wphase<CT, 2, false, KW, true>};
   for (const void *f : fns) {
     hipError_t e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, max_lds);
     if (e != hipSuccess) return e;
@@ -439,9 +468,11 @@ static hipError_t configure_wphase_k(int max_lds) {
 
 template <typename CT, int KP>
 static hipError_t configure_phase_k(int max_lds) {
-  const void *fns[] = {(const void *)k_phase<CT, 0, true, KP>,  (const void *)k_phase<CT, 0, false, KP>,
-                       (const void *)k_phase<CT, 1, true, KP>,  (const void *)k_phase<CT, 1, false, KP>,
-                       (const void *)k_phase<CT, 2, true, KP>,  (const void *)k_phase<CT, 2, false, KP>};
+  const void *fns[] = {(const void *)k_phase<CT, 0, true, KP, false>, (const void *)k_phase<CT, 0, false, KP, false>,
+                       (const void *)k_phase<CT, 1, true, KP, false>, (const void *)k_phase<CT, 1, false, KP, false>,
+                       (const void *)k_phase<CT, 2, true, KP, false>, (const void *)k_phase<CT, 2, false, KP, false>,
+                       (const void *)k_phase<CT, 1, true, KP, true>,  (const void *)k_phase<CT, 1, false, KP, true>,
+                       (const void *)k_phase<CT, 2, true, KP, true>,  (const void *)k_phase<CT, 2, false, KP, true>};
   for (const void *f : fns) {
     hipError_t e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, max_lds);
     if (e != hipSuccess) return e;

@@ -379,10 +379,10 @@ __device__ __forceinline__ TendPoint tend_segment(const Args &a, const Member &m
 }
 
 // Row tile t = (member, row, segment of kSeg longitudes) of a phase launch.
-// FUSED = false (k_tend): rows 0..M-1; components of flagged rows are
-// staged to HBM for the filter kernel, which finishes their epilogue.
-// FUSED = true (k_phase): rows from the far-row ranges; flagged components
-// are left to the launch's whole-row filter tiles.
+// The rows are those of the launch's row ranges.  FUSED = false (k_tend):
+// components of flagged rows are staged to HBM for the filter kernel, which
+// finishes their epilogue.  FUSED = true (k_phase): flagged components are
+// left to the launch's whole-row filter tiles.
 __device__ __forceinline__ int far_row(const Args &a, int r) {
 #pragma unroll
   for (int k = 0; k < kMaxFarRng; ++k) {
@@ -404,10 +404,10 @@ template <typename CT, int PASS, bool IN_FULL, bool FUSED>
 __device__ __forceinline__ void tend_tile(const Args &a, int t, unsigned char *smem, double *red, bool bar2 = false,
                                           bool live = true) {
   const int M = a.M, P = a.pitch, nseg = a.nseg, tid = ltid();
-  const int nrows = FUSED ? a.nfar_rows : M;
+  const int nrows = a.nfar_rows;
   const int mloc = t / (nrows * nseg), rem = t - mloc * (nrows * nseg);
   const int r = rem / nseg, g = rem - (rem / nseg) * nseg;
-  const int j = FUSED ? far_row(a, r) : r;
+  const int j = far_row(a, r);
   const Member mb = member_at(a, a.m0 + mloc);
   const RowCoef cj = a.coef[j];
   const bool has_u = j >= 1 && j <= M - 2, has_v = j <= M - 2;

@@ -412,9 +412,13 @@ enum { GD_TIME_TEND = 0, GD_TIME_FILTER = 1, GD_TIME_UPDATE = 2, GD_TIME_PHASE =
  * tiles stay within 24576 (num_lon <= 1024) or 6144 (num_lon <= 2048), in
  * form 2 for rows of 255 to 508 longitudes while its workgroups (filtered
  * rows plus far rows) fit two per compute unit; gd_autotune may choose any
- * form.  GD_FUSED=0, 1 or 2 in the environment when the handle is created
- * forces a form (2 falls back to 1 outside 255 to 762 longitudes).  Every
- * form gives the same bits.  No counterpart in the reference. */
+ * form.  In the calls of csp2 the rows away from the polar filter run as strip
+ * tiles (several rows each) beside the launch's other rows, and the form is
+ * then chosen by its filtered rows.
+ * GD_FUSED=0, 1 or 2 in the environment when the handle is created forces a
+ * form (2 falls back to 1 outside 255 to 762 longitudes); GD_STRIP=n gives the
+ * rows per strip tile (0: none).  Every form gives the same bits.  No
+ * counterpart in the reference. */
 int gd_fused_phases(const gd_handle *h);
 
 /* Tile autotuner (no counterpart in the reference).  For the current
