@@ -83,6 +83,8 @@ struct gd_handle {
   StageSlot *dslots = nullptr;
   std::vector<FiltRow> frows;    // filter workgroups: (member, latitude) with staged rows
   FiltRow *dfrows = nullptr;
+  std::vector<FiltGroup> fgroups;  // the filtered rows of one member
+  FiltGroup *dfgroups = nullptr;
   std::vector<int32_t> mslots;   // staging slots of the momentum rows (MFMA filter)
   int32_t *dmslots = nullptr;
   void *dmm_phi = nullptr;       // basis matrices of the MFMA filter
@@ -93,9 +95,10 @@ struct gd_handle {
   // fused phase launches (k_phase): the filter rows inside the tendency
   // launch; the row tiles cover the row ranges far_lo/far_cnt.  fused_ok:
   // the shape allows them; wide_ok: also workgroups of two tiles (k_wphase);
-  // fused_mode: -1 by launch size, 0 never, 1 always k_phase, 2 always
-  // k_wphase where wide_ok
-  bool fused_ok = false, wide_ok = false;
+  // rphase_ok: also one workgroup per filtered row (k_rphase, calls with strip
+  // tiles only); fused_mode: -1 by launch size, 0 never, 1 always k_phase, 2
+  // always k_wphase where wide_ok, 3 k_rphase where a call can take it
+  bool fused_ok = false, wide_ok = false, rphase_ok = false;
   int fused_mode = -1;
   int upd_narrow = -1;  // k_update rounds of four points and partials per thread: -1 by band size, 0 no, 1 yes
   int ncu = 256;  // compute units of the device
@@ -180,6 +183,9 @@ Args base_args(const gd_handle *h) {
   a.coef = h->dcoef;
   a.slots = h->dslots;
   a.frows = h->dfrows;
+  a.fgroups = h->dfgroups;
+  a.nfgroup = (int)h->fgroups.size();
+  a.nfrow = (int)(h->frows.size() / h->nmem);
   a.twid = h->dtwid;
   a.ghost = h->dghost;
   a.fft_L = h->fft_L;
@@ -297,10 +303,10 @@ constexpr int64_t kFusedMaxTilesWide = 6144;
 // asked for or tuned.
 int phase_form(const gd_handle *h) {
   if (!h->fused_ok || h->fused_mode == 0) return 0;
-  if (h->fused_mode == 1) return 1;
+  if (h->fused_mode == 1 || h->fused_mode == 3) return 1;
   if (h->fused_mode == 2) return h->wide_ok ? 2 : 1;
   auto it = h->tuned_fused.find(h->nact);
-  if (it != h->tuned_fused.end()) return it->second == 2 && !h->wide_ok ? 1 : it->second;
+  if (it != h->tuned_fused.end()) return it->second == 3 || (it->second == 2 && !h->wide_ok) ? 1 : it->second;
   if (h->wide_ok && (h->N + kSeg - 1) / kSeg == 2) {
     const int64_t wgs = (int64_t)h->nact * ((int64_t)(h->frows.size() / h->nmem) + h->far.rows);
     if (wgs <= 2 * (int64_t)h->ncu) return 2;
@@ -324,12 +330,21 @@ int strip_rows(const gd_handle *h) {
 }
 
 // Form of the phase launches of a call with strip tiles, unless the handle's
-// form is forced or tuned: k_wphase (shortest chain of a filter row) while its
-// workgroups fit about two per CU, else k_phase.  Measured on MI355X, ms per
-// step: 360x181 0.241 against 0.267 (k_phase), four of them 0.326 / 0.341,
-// 720x361 0.355 / 0.366; 0.533 / 0.461 for two of 720x361.
+// form is forced or tuned: 1 k_phase, 2 k_wphase, 3 k_rphase.
+// k_wphase (shortest chain of a filter row) while its workgroups fit about two
+// per CU: 360x181 0.241 ms per step against 0.267 (k_phase) and 0.327
+// (k_rphase), four of them 0.326 / 0.341 / 0.395, 720x361 0.355 / 0.366 /
+// 0.539; 0.533 / 0.461 / 0.597 for two of 720x361.  k_rphase (most rows in
+// flight) once its filtered rows fill the CUs: 8 of 360x181 0.476 / 0.520
+// (k_phase), 16 of 180x91 0.336 / 0.340, 64 of them 0.804 / 1.009, 4 of
+// 720x361 0.703 / 0.713, 64 of 360x181 3.34 / 3.69; but 0.305 / 0.279 for 8
+// of 180x91, and 1.55 / 1.49 for 4 of 1000x501, where a lane's 16 longitudes
+// spill.
 int strip_form(const gd_handle *h) {
-  if (!h->fused_ok || h->fused_mode >= 0 || h->tuned_fused.count(h->nact)) return phase_form(h);
+  if (h->fused_mode == 3 && h->rphase_ok) return 3;
+  const auto it = h->tuned_fused.find(h->nact);
+  if (it != h->tuned_fused.end() && it->second == 3 && h->rphase_ok) return 3;
+  if (!h->fused_ok || h->fused_mode >= 0 || it != h->tuned_fused.end()) return phase_form(h);
   const int64_t nact = h->nact, nseg = (h->N + kSeg - 1) / kSeg;
   if (h->wide_ok) {
     const int64_t R = strip_rows(h), groups = (h->strip_b - h->strip_a + R) / R;
@@ -337,6 +352,7 @@ int strip_form(const gd_handle *h) {
                         (nact * nseg * (h->near_far.rows + groups) + 1) / 2;
     if (10 * wgs <= 22 * (int64_t)h->ncu) return 2;
   }
+  if (h->rphase_ok && h->N <= 768 && 8 * nact * (int64_t)h->fgroups.size() >= 7 * (int64_t)h->ncu) return 3;
   return 1;
 }
 
@@ -355,6 +371,7 @@ hipError_t enqueue_phase(gd_handle *h, Args a, int pass, bool in_full, bool stri
     return enqueue_filter(h, a);
   }
   set_fused(h, a, h->nact, strip ? h->near_far : h->far);
+  if (form == 3) return run(h, "phase", [&] { return launch_rphase(a, h->prec, pass, in_full, h->stream); });
   if (form == 2) return run(h, "wphase", [&] { return launch_wphase(a, h->prec, pass, in_full, h->stream); });
   return run(h, "phase", [&] { return launch_phase(a, h->prec, pass, in_full, h->stream); });
 }
@@ -635,6 +652,11 @@ void build_tables(gd_handle *h, std::vector<RowCoef> &rc) {
       f.wrow = ss.comp == CDV ? rc[ss.row].hcos : rc[ss.row].fcos;
       h->frows.push_back(f);
     }
+  h->fgroups.clear();
+  for (size_t k = 0; k < order.size(); ++k) {
+    if (!k || h->slots[order[k]].row != h->slots[order[k - 1]].row) h->fgroups.push_back(FiltGroup{(int32_t)k, 0});
+    ++h->fgroups.back().n;
+  }
 }
 
 // Radix passes of the complex FFT of length L: 8s first, then 4, 2, 3, 5,
@@ -925,7 +947,7 @@ int gd_create(const gd_config *cfg, int32_t n_members, gd_handle **out) {
       }
     }
     const char *env = std::getenv("GD_FUSED");
-    h->fused_mode = env && env[0] >= '0' && env[0] <= '2' ? env[0] - '0' : -1;
+    h->fused_mode = env && env[0] >= '0' && env[0] <= '3' ? env[0] - '0' : -1;
     const char *bd = std::getenv("GD_STRIP");
     if (bd && bd[0]) h->strip_mode = std::max(0, std::min(std::atoi(bd), 32));
     const char *nar = std::getenv("GD_UPD_NARROW");
@@ -935,6 +957,8 @@ int gd_create(const gd_config *cfg, int32_t n_members, gd_handle **out) {
                   phase_lds_bytes(h->N, h->fft_L, h->prec) <= prop.sharedMemPerBlock;
     const int nseg = (h->N + kSeg - 1) / kSeg;
     h->ncu = prop.multiProcessorCount > 0 ? prop.multiProcessorCount : 256;
+    h->rphase_ok = h->fused_ok && h->N <= 4 * kBlock &&
+                   rphase_lds_bytes(h->N, h->fft_L, h->prec) <= prop.sharedMemPerBlock;
     h->wide_ok = h->fused_ok && (nseg == 2 || nseg == 3) &&
                  wphase_lds_bytes(h->N, h->fft_L, h->prec) <= prop.sharedMemPerBlock;
   }
@@ -969,6 +993,7 @@ int gd_create(const gd_config *cfg, int32_t n_members, gd_handle **out) {
   h->dcoef = (RowCoef *)dalloc(h, sizeof(RowCoef) * h->M, e);
   h->dslots = (StageSlot *)dalloc(h, sizeof(StageSlot) * std::max<size_t>(nslots, 1), e);
   h->dfrows = (FiltRow *)dalloc(h, sizeof(FiltRow) * std::max<size_t>(h->frows.size(), 1), e);
+  h->dfgroups = (FiltGroup *)dalloc(h, sizeof(FiltGroup) * std::max<size_t>(h->fgroups.size(), 1), e);
   h->dtwid = (double *)dalloc(h, (size_t)tw_padded(h->N) * 2 * 8, e);
   h->dstep = (int32_t *)dalloc(h, sizeof(int32_t) * h->nmem, e);
   h->dghost = (double *)dalloc(h, (size_t)2 * h->P * 8, e);
@@ -1001,7 +1026,7 @@ int gd_create(const gd_config *cfg, int32_t n_members, gd_handle **out) {
   std::vector<unsigned char> strip_tab;
   strip_rows_fill(rc, h->prec, strip_tab);
   h->dstrip = dalloc(h, strip_tab.size(), e);
-  if (!h->dstrip || !h->ddiag || !h->dcoef || !h->dslots || !h->dfrows || !h->dtwid ||
+  if (!h->dstrip || !h->ddiag || !h->dcoef || !h->dslots || !h->dfrows || !h->dfgroups || !h->dtwid ||
       !h->dstep || !h->dghost || !h->dprow[0] || !h->dprow[1] || !h->dmslots) {
     gd_destroy(h);
     return fail(nullptr, GD_ERR_HIP, "device allocation failed");
@@ -1020,6 +1045,9 @@ int gd_create(const gd_config *cfg, int32_t n_members, gd_handle **out) {
   if (nslots) hipMemcpyAsync(h->dslots, h->slots.data(), sizeof(StageSlot) * nslots, hipMemcpyHostToDevice, h->stream);
   if (!h->frows.empty())
     hipMemcpyAsync(h->dfrows, h->frows.data(), sizeof(FiltRow) * h->frows.size(), hipMemcpyHostToDevice, h->stream);
+  if (!h->fgroups.empty())
+    hipMemcpyAsync(h->dfgroups, h->fgroups.data(), sizeof(FiltGroup) * h->fgroups.size(), hipMemcpyHostToDevice,
+                   h->stream);
   hipMemcpyAsync(h->dtwid, tw.data(), tw.size() * 8, hipMemcpyHostToDevice, h->stream);
   if (!h->mslots.empty())
     hipMemcpyAsync(h->dmslots, h->mslots.data(), sizeof(int32_t) * h->mslots.size(), hipMemcpyHostToDevice,
@@ -1398,7 +1426,8 @@ int gd_autotune(gd_handle *h, int32_t steps, const char *cache_path, int32_t *fu
   double bms = 0.0;
   if (cache_path && !cache_path[0]) cache_path = nullptr;  // "" : no cache
   bool cached = cache_path && tune_lookup(cache_path, key, bf, bw, bms);
-  if (cached && (bw < 1 || bw > h->M || bf < 0 || bf > 2 || (bf && !h->fused_ok) || (bf == 2 && !h->wide_ok)))
+  if (cached && (bw < 1 || bw > h->M || bf < 0 || bf > 3 || (bf && !h->fused_ok) || (bf == 2 && !h->wide_ok) ||
+                 (bf == 3 && !h->rphase_ok)))
     cached = false;
   if (!cached) {
     // fused or separate phase launches (both give the same bits; a forced
@@ -1410,6 +1439,8 @@ int gd_autotune(gd_handle *h, int32_t steps, const char *cache_path, int32_t *fu
       fopts = {0, 1, 2};
     else
       fopts = {0, 1};
+    if (h->fused_mode < 0 && h->rphase_ok && h->strip_b >= h->strip_a && h->cfg.split_scheme == GD_SPLIT_CSP2)
+      fopts.push_back(3);
     // ... and k_update rows per workgroup (each workgroup forms its member's
     // beta from all of the member's partials in one order: the same bits)
     std::vector<int> wopts;

@@ -85,6 +85,17 @@ __device__ __forceinline__ void wave_sums_to(const double (&v)[K], double *dst) 
   }
 }
 
+// One wave holding a whole row: v[k] are the values of the lanes of wave k of a
+// tile; their total as block_sum adds it, the same in every lane.
+__device__ __forceinline__ double row_total(const double (&v)[4]) {
+  const double s = fold_row(fold16(fold32(v[0], v[1]), fold32(v[2], v[3])));
+  auto at = [s](int lane) {
+    return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(s), lane),
+                            __builtin_amdgcn_readlane(__double2loint(s), lane));
+  };
+  return ((at(0) + at(32)) + at(16)) + at(48);
+}
+
 // Deterministic sum over the kBlock threads of a tile (fixed butterfly +
 // fixed cross-wave order); every thread of the tile returns the same value.
 // The barriers are the workgroup's, so every tile of a workgroup calls it
@@ -114,6 +125,10 @@ __device__ __forceinline__ void block_sum_n(double (&v)[K], double *red) {
     for (int k = 1; k < kBlock / 64; ++k) s += red[k * K + q];
     v[q] = s;
   }
+}
+
+__device__ __forceinline__ const double *fld_ptr(const Member &mb, int slot, int comp) {
+  return mb.st(slot, comp == CDU ? FU : (comp == CDV ? FV : FGD));
 }
 
 __device__ __forceinline__ double fld_base(const Member &mb, int slot, int comp, size_t o) {

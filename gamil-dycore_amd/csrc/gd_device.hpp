@@ -102,6 +102,12 @@ struct FiltRow {
   double wrow;      // area weight of the row in the beta inner products
 };
 
+// The filtered components of one row: entries first .. first + n - 1 of a
+// member's filter rows (n <= 3, components in order).
+struct FiltGroup {
+  int32_t first, n;
+};
+
 struct Args {
   char *arena;                 // member m at arena + m * mstride
   size_t mstride, fs, cs, off_part, off_dpart, off_sx, off_beta, off_sy;
@@ -109,6 +115,8 @@ struct Args {
   const RowCoef *coef;
   const StageSlot *slots;
   const FiltRow *frows;
+  const FiltGroup *fgroups;    // k_rphase: the filtered rows of a member ...
+  int nfgroup, nfrow;          // ... their number, and a member's filter rows
   const int32_t *mslots;       // k_filter_mm: the staging slots of the momentum rows
   const void *mm_phi;          // k_filter_mm: the basis matrices (mm_basis_fill)
   int mm;                      // k_filter: momentum rows come projected in sy (MFMA modes)

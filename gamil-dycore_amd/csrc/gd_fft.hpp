@@ -134,6 +134,24 @@ __device__ __forceinline__ void dft_small(double2 (&v)[R], Tw tw, int rstep, boo
   }
 }
 
+// Thread index and synchronisation of the NT threads that transform a row: a
+// workgroup (barrier), or with NT = 64 a single wave, whose LDS accesses are in
+// order, so only the compiler is held to it.
+template <int NT>
+__device__ __forceinline__ int fft_tid() {
+  return NT == 64 ? (int)(threadIdx.x & 63) : (int)threadIdx.x;
+}
+template <int NT>
+__device__ __forceinline__ void fft_sync() {
+  if constexpr (NT == 64) {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  } else {
+    __syncthreads();
+  }
+}
+
 // One Stockham pass of radix R over a row of L points: butterfly j reads
 // points j + q L/R, twiddles them by W_{Ns R}^{q (j mod Ns)} and writes its
 // outputs to ((j - j mod Ns) R + j mod Ns) + q Ns.
@@ -157,7 +175,7 @@ __device__ __forceinline__ void fft_pass(const double2 *src, double2 *dst, int L
   const unsigned Lr = L / R;
   const int tws = (L / (Ns * R)) * tstride;
   const int rstep = (int)Lr * tstride;
-  for (unsigned j = threadIdx.x; j < Lr; j += NT) {
+  for (unsigned j = fft_tid<NT>(); j < Lr; j += NT) {
     const unsigned k = j % (unsigned)Ns;
     double2 v[R];
 #pragma unroll
@@ -180,7 +198,7 @@ __device__ __forceinline__ void fft_pass_any(const double2 *src, double2 *dst, i
   const int Lr = L / R;
   const int tws = (L / (Ns * R)) * tstride;
   const int rstep = Lr * tstride;
-  for (int j = threadIdx.x; j < Lr; j += NT) {
+  for (int j = fft_tid<NT>(); j < Lr; j += NT) {
     const int k = j % Ns;
     const int o = (j - k) * R + k;
     for (int q = 0; q < R; ++q) {
@@ -213,7 +231,7 @@ __device__ __forceinline__ int fft_run(double2 *b0, double2 *b1, int cur, const 
       case 8: fft_pass<8, false, false, NT>(src, dst, L, Ns, tw, tstride, inv); break;
       default: fft_pass_any<NT>(src, dst, L, Ns, R, tw, tstride, inv); break;
     }
-    __syncthreads();
+    fft_sync<NT>();
     Ns *= R;
     cur ^= 1;
   }
@@ -231,7 +249,7 @@ template <int NT, int L, int TS, int NS, bool SWI, int R, int... REST>
 __device__ __forceinline__ int fft_fixed_p(double2 *b0, double2 *b1, int cur, Tw tw, bool inv) {
   constexpr bool SWO = NS == 1 && R == 8 && L % 8 == 0 && sizeof...(REST) > 0;
   fft_pass<R, SWI, SWO, NT>(cur ? b1 : b0, cur ? b0 : b1, L, NS, tw, TS, inv);
-  __syncthreads();
+  fft_sync<NT>();
   if constexpr (sizeof...(REST) > 0)
     return fft_fixed_p<NT, L, TS, NS * R, SWO, REST...>(b0, b1, cur ^ 1, tw, inv);
   else
@@ -275,7 +293,7 @@ __device__ __forceinline__ double2 fmask(double2 X, int k, int c) {
 template <int NT = kBlock>
 __device__ __forceinline__ void real_mid(const double2 *s, double2 *d, int L, int c, Tw tw, double sc) {
   const int H = L / 2 + 1;
-  for (int k = threadIdx.x; k < H; k += NT) {
+  for (int k = fft_tid<NT>(); k < H; k += NT) {
     if (k == 0) {
       const double2 z = s[0];
       const double X0 = z.x + z.y, XL = z.x - z.y;
@@ -303,7 +321,7 @@ __device__ __forceinline__ void real_mid(const double2 *s, double2 *d, int L, in
 // Odd N: mask the full complex spectrum symmetrically, scaled by 1/N.
 template <int NT = kBlock>
 __device__ __forceinline__ void cplx_mid(const double2 *s, double2 *d, int L, int c, double sc) {
-  for (int k = threadIdx.x; k < L; k += NT) {
+  for (int k = fft_tid<NT>(); k < L; k += NT) {
     const int kk = k <= L - k ? k : L - k;
     const double2 Y = fmask(s[k], kk, c);
     d[k] = make_double2(Y.x * sc, Y.y * sc);
@@ -615,6 +633,95 @@ __device__ __forceinline__ void filter_row_w(const Args &a, const Member &mb, co
     }
   }
   __syncthreads();  // LDS free for the caller
+}
+
+// filter_row<CT, KP, true> (the row already in b0, a rescaled phase) by one
+// wave with KQ longitudes per lane (l = lane + 64 q, N <= 64 KQ): no barrier,
+// so the waves of a workgroup filter different rows.  The sums keep
+// filter_row's order: lane l adds the products of longitudes l + 64 v, l + 64 v
+// + kBlock, ... as its thread l + 64 v does, the four sums over the lanes are
+// its four waves', added in turn.
+template <typename CT, int KQ>
+__device__ __forceinline__ void filter_wave(const Args &a, const Member &mb, const FiltRow &fr, double2 *tw,
+                                            double2 *b0, double2 *b1, bool zero) {
+  const int N = a.N, L = a.fft_L, lane = threadIdx.x & 63;
+  const double sc = 1.0 / (double)L;
+  const int comp = fr.comp;
+  const size_t o = (size_t)fr.row * a.pitch;
+  const int ystep = a.fft_half ? 1 : 2;
+  const double *wp = mb.st(a.s_in, comp == CDU ? FU : (comp == CDV ? FV : FGD)) + o;
+  const double *wq = (comp == CDGD ? mb.ghs() : mb.st(a.s_in, FGD)) + o;
+  const double *pp = (a.phase == PH_C ? mb.tb(comp) : fld_ptr(mb, a.s0, comp)) + o;
+  double x[KQ], w[KQ], pre[KQ], yv[KQ];
+#pragma unroll
+  for (int q = 0; q < KQ; ++q) {
+    const int l = lane + 64 * q, lc = l < N ? l : 0;
+    x[q] = zero ? 0.0 : ((const double *)b0)[(size_t)lc * ystep];
+    yv[q] = 0.0;
+  }
+  // the rescale weights (state%iap%u, %v, gd + ghs) and epilogue inputs are
+  // issued between the transforms: held from there on, they leave the forward
+  // transform its registers, and the inverse one covers their latency
+  auto late = [&] {
+#pragma unroll
+    for (int q = 0; q < KQ; ++q) {
+      const int l = lane + 64 * q, lc = l < N ? l : 0;
+      if (!zero) {
+        w[q] = wp[lc];
+        if (comp == CDGD) w[q] = w[q] + wq[lc];
+      }
+      pre[q] = pp[lc];
+    }
+  };
+  double s1 = 0.0, s2 = 0.0;
+  if (!zero) {
+    const Tw twt{tw, N};
+    fft_sync<64>();
+    int cur = fft_any<4, 64>(b0, b1, 0, a, twt, false);
+    if (a.fft_half)
+      real_mid<64>(cur ? b1 : b0, cur ? b0 : b1, L, fr.cut, twt, sc);
+    else
+      cplx_mid<64>(cur ? b1 : b0, cur ? b0 : b1, L, fr.cut, sc);
+    late();
+    fft_sync<64>();
+    cur = fft_any<4, 64>(b0, b1, cur ^ 1, a, twt, true);
+    const double *y = (const double *)(cur ? b1 : b0);
+    double a1[4] = {0, 0, 0, 0}, a2[4] = {0, 0, 0, 0};
+#pragma unroll
+    for (int q = 0; q < KQ; ++q) {
+      const int l = lane + 64 * q;
+      if (l < N) {
+        yv[q] = y[(size_t)l * ystep];
+        a1[q & 3] += x[q] * w[q];
+        a2[q & 3] += yv[q] * w[q];
+      }
+    }
+    s1 = row_total(a1);
+    s2 = row_total(a2);
+  } else {
+    late();
+  }
+  // rows with |s1| <= filter_inner_product_threshold stay unfiltered
+  const bool filt = fabs(s1) > 1.0e-16;
+  double p1[4] = {0, 0, 0, 0}, p2[4] = {0, 0, 0, 0};
+#pragma unroll
+  for (int q = 0; q < KQ; ++q) {
+    const int l = lane + 64 * q;
+    if (l < N) {
+      const double T = filt ? yv[q] * s1 / s2 : x[q];
+      phase_store<CT>(a, mb, comp, o + l, T, pre[q], fr.wrow, p1[q & 3], p2[q & 3]);
+    }
+  }
+  if (a.phase == PH_C) {
+    const double t1 = row_total(p1), t2 = row_total(p2);
+    // the whole row's products go to segment 0 of its partials, the other
+    // segments of the row hold zero
+    double *part = mb.part() + ((size_t)(fr.row * 3 + comp) * a.nseg) * 2;
+    if (lane < a.nseg) {
+      part[2 * lane] = lane == 0 ? t1 : 0.0;
+      part[2 * lane + 1] = lane == 0 ? t2 : 0.0;
+    }
+  }
 }
 
 inline size_t filter_lds_bytes_h(int N, int L) { return (size_t)tw_entries(N) * 16 + (size_t)2 * L * 16; }

@@ -69,6 +69,10 @@ size_t phase_lds_bytes(int N, int L, int prec);
 // of two or three segments; a.ntiles counts segment tiles as for launch_phase
 hipError_t launch_wphase(const Args &a, int prec, int pass, bool in_full, hipStream_t s);
 size_t wphase_lds_bytes(int N, int L, int prec);
+// a fast or slow phase with one workgroup per filtered row (k_rphase,
+// gd_phase.hip); num_lon <= 1024
+hipError_t launch_rphase(const Args &a, int prec, int pass, bool in_full, hipStream_t s);
+size_t rphase_lds_bytes(int N, int L, int prec);
 // momentum rows of the filter as batched MFMA products (gd_filter_mm.hip):
 // one workgroup per (momentum slot in a.mslots, block of 16 members)
 hipError_t launch_filter_mm(const Args &a, bool bf16, hipStream_t s);

@@ -303,6 +303,88 @@ k_wphase(const Args a) {
 }
 
 // ---------------------------------------------------------------------------
+// k_rphase: k_phase with one workgroup per filtered row (up to three
+// components) instead of one per row and component.  The workgroup evaluates
+// the row's tendencies once, then each component is filtered by one wave
+// (filter_wave): the transforms keep at most 45 to 120 butterflies busy per
+// pass, one or two waves' worth, so four waves behind a barrier per pass mostly
+// wait, where here every resident wave has a row of its own.
+//
+// LDS: [stencil rows, later the three components' FFT buffers b1] [their row
+// buffers b0] [twiddle table].
+// ---------------------------------------------------------------------------
+
+template <typename CT>
+__host__ __device__ inline size_t rphase_region0(int L) {
+  const size_t st = tend_stencil_bytes<CT>(), fb = (size_t)3 * L * 16;
+  return align16(st > fb ? st : fb);
+}
+
+template <typename CT>
+__host__ __device__ inline size_t rphase_lds(int N, int L) {
+  return rphase_region0<CT>(L) + (size_t)3 * L * 16 + (size_t)tw_padded(N) * 16;
+}
+
+template <typename CT, int PASS, bool IN_FULL, int KQ>
+__device__ __forceinline__ void rnear_block(const Args &a, int t, unsigned char *smem, double *red) {
+  const int N = a.N, L = a.fft_L, tid = threadIdx.x;
+  const FiltGroup fg = a.fgroups[t % a.nfgroup];
+  const FiltRow *fr0 = a.frows + (size_t)(t / a.nfgroup) * a.nfrow + fg.first;
+  const Member mb = member_at(a, fr0->member);
+  const int j = fr0->row;
+  const RowCoef cj = a.coef[j];
+  double2 *b1 = (double2 *)smem;
+  double2 *b0 = (double2 *)(smem + rphase_region0<CT>(L));
+  double2 *tw = b0 + 3 * L;
+  tw_to_lds(a, tw);
+  constexpr int CM = TC_DU | TC_DV | (PASS != 2 ? TC_DGD : 0);
+  const RowNbr nb = row_nbr(a, j);
+  SegLoads cur;
+  seg_load<PASS, IN_FULL>(a, mb, j, 0, min(N, kSeg), cur);
+  for (int g = 0; g < a.nseg; ++g) {
+    const int i0 = g * kSeg, W = min(N - i0, kSeg);
+    SegLoads nxt;
+    if (g + 1 < a.nseg) seg_load<PASS, IN_FULL>(a, mb, j, i0 + kSeg, min(N - i0 - kSeg, kSeg), nxt);
+    if (g) __syncthreads();  // the previous segment's stencil rows have been read
+    const TendPoint pt = seg_eval<CT, PASS, IN_FULL, CM>(a, cj, nb, j, i0, W, cur, false, 0.0,
+                                                         TendPoint{0, 0, 0, 0, 0, 0}, smem, red);
+    if (tid < W) {
+      row_put(a, (double *)(b0 + CDU * L), i0 + tid, pt.du);
+      row_put(a, (double *)(b0 + CDV * L), i0 + tid, pt.dv);
+      if (PASS != 2) row_put(a, (double *)(b0 + CDGD * L), i0 + tid, pt.dgd);
+    }
+    cur = nxt;
+  }
+  __builtin_amdgcn_s_waitcnt(0);  // the twiddle copy has landed
+  __syncthreads();  // rows and twiddles published; the stencil rows are free for b1
+  const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+  if (wv >= fg.n) return;
+  const FiltRow fr = fr0[wv];
+  // (the slow pass has no mass continuity term: its dgd rows are zero rows)
+  filter_wave<CT, KQ>(a, mb, fr, tw, b0 + fr.comp * L, b1 + fr.comp * L, PASS == 2 && fr.comp == CDGD);
+}
+
+template <typename CT, int PASS, bool IN_FULL, int KQ>
+__global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(KQ == 8 ? 4 : 3, 8)))
+k_rphase(const Args a) {
+  extern __shared__ __align__(16) unsigned char smem[];
+  __shared__ double red[4 * 6];
+  const int b = blockIdx.x;
+  if (b < a.nnear_pad) {
+    const int t = (b % kXcd) * (a.nnear_pad / kXcd) + b / kXcd;
+    if (t < a.nnear) rnear_block<CT, PASS, IN_FULL, KQ>(a, t, smem, red);
+    return;
+  }
+  if (b >= a.nnear_pad + a.row_blk) {
+    strip_block<CT, PASS, IN_FULL>(a, a.nnear_pad + a.row_blk, smem);
+    return;
+  }
+  const int bb = b - a.nnear_pad, t = (bb % kXcd) * (a.row_blk / kXcd) + bb / kXcd;
+  if (t >= a.ntiles) return;
+  tend_tile<CT, PASS, IN_FULL, true>(a, t, smem, red);
+}
+
+// ---------------------------------------------------------------------------
 // k_dphase: the last application of ordinary_diffusion with its filter rows
 // (diffusion_mod.F90:74-217 and the filter of dycore_mod.F90:658-666) in one
 // launch, in place of k_diffuse followed by k_filter; same bits.
@@ -421,6 +503,45 @@ hipError_t launch_phase(const Args &a, int prec, int pass, bool in_full, hipStre
   return prec == 0 ? launch_phase_k<double, 4>(a, pass, in_full, s) : launch_phase_k<float, 4>(a, pass, in_full, s);
 }
 
+template <typename CT, int KQ>
+static hipError_t launch_rphase_k(Args a, int pass, bool in_full, hipStream_t s) {
+  a.nnear = a.nnear / a.nfrow * a.nfgroup;
+  a.nnear_pad = pad_xcd(a.nnear);
+  a.row_blk = pad_xcd(a.ntiles);
+  a.strip_blk = strip_blocks(a, 1);
+  dim3 g(a.nnear_pad + a.row_blk + a.strip_blk), b(kBlock);
+  const size_t lds = rphase_lds<CT>(a.N, a.fft_L);
+#define GD_PH(P, F) hipLaunchKernelGGL((k_rphase<CT, P, F, KQ>), g, b, lds, s, a)
+  if (pass == 1) { if (in_full) GD_PH(1, true); else GD_PH(1, false); }
+  else { if (in_full) GD_PH(2, true); else GD_PH(2, false); }
+#undef GD_PH
+  return hipGetLastError();
+}
+
+hipError_t launch_rphase(const Args &a, int prec, int pass, bool in_full, hipStream_t s) {
+  if (a.N > 1024 || pass < 1 || pass > 2 || a.phase > PH_C) return hipErrorInvalidValue;
+  if (a.N > 512 && a.N <= 768)
+    return prec == 0 ? launch_rphase_k<double, 12>(a, pass, in_full, s) : launch_rphase_k<float, 12>(a, pass, in_full, s);
+  if (a.N <= 512)
+    return prec == 0 ? launch_rphase_k<double, 8>(a, pass, in_full, s) : launch_rphase_k<float, 8>(a, pass, in_full, s);
+  return prec == 0 ? launch_rphase_k<double, 16>(a, pass, in_full, s) : launch_rphase_k<float, 16>(a, pass, in_full, s);
+}
+
+size_t rphase_lds_bytes(int N, int L, int prec) {
+  return prec == 0 ? rphase_lds<double>(N, L) : rphase_lds<float>(N, L);
+}
+
+template <typename CT, int KQ>
+static hipError_t configure_rphase_k(int max_lds) {
+  const void *fns[] = {(const void *)k_rphase<CT, 1, true, KQ>, (const void *)k_rphase<CT, 1, false, KQ>,
+                       (const void *)k_rphase<CT, 2, true, KQ>, (const void *)k_rphase<CT, 2, false, KQ>};
+  for (const void *f : fns) {
+    hipError_t e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, max_lds);
+    if (e != hipSuccess) return e;
+  }
+  return hipSuccess;
+}
+
 template <typename CT, int KW>
 static hipError_t launch_wphase_k(Args a, int pass, bool in_full, hipStream_t s) {
   a.row_blk = pad_xcd((a.ntiles + kWTiles - 1) / kWTiles);  // row workgroups
@@ -486,6 +607,12 @@ hipError_t configure_phase(int max_lds) {
   if ((e = configure_phase_k<float, 4>(max_lds)) != hipSuccess) return e;
   if ((e = configure_phase_k<double, 8>(max_lds)) != hipSuccess) return e;
   if ((e = configure_phase_k<float, 8>(max_lds)) != hipSuccess) return e;
+  if ((e = configure_rphase_k<double, 8>(max_lds)) != hipSuccess) return e;
+  if ((e = configure_rphase_k<float, 8>(max_lds)) != hipSuccess) return e;
+  if ((e = configure_rphase_k<double, 12>(max_lds)) != hipSuccess) return e;
+  if ((e = configure_rphase_k<float, 12>(max_lds)) != hipSuccess) return e;
+  if ((e = configure_rphase_k<double, 16>(max_lds)) != hipSuccess) return e;
+  if ((e = configure_rphase_k<float, 16>(max_lds)) != hipSuccess) return e;
   if ((e = configure_wphase_k<double, 1>(max_lds)) != hipSuccess) return e;
   if ((e = configure_wphase_k<float, 1>(max_lds)) != hipSuccess) return e;
   if ((e = configure_wphase_k<double, 2>(max_lds)) != hipSuccess) return e;

@@ -414,9 +414,11 @@ enum { GD_TIME_TEND = 0, GD_TIME_FILTER = 1, GD_TIME_UPDATE = 2, GD_TIME_PHASE =
  * rows plus far rows) fit two per compute unit; gd_autotune may choose any
  * form.  In the calls of csp2 the rows away from the polar filter run as strip
  * tiles (several rows each) beside the launch's other rows, and the form is
- * then chosen by its filtered rows.
- * GD_FUSED=0, 1 or 2 in the environment when the handle is created forces a
- * form (2 falls back to 1 outside 255 to 762 longitudes); GD_STRIP=n gives the
+ * then chosen by its filtered rows: 2, 1, or one fused launch with a workgroup
+ * per filtered row (num_lon <= 1024), which this function reports as 1.
+ * GD_FUSED=0, 1, 2 or 3 in the environment when the handle is created forces
+ * a form (2 falls back to 1 outside 255 to 762 longitudes; 3, the workgroup
+ * per filtered row, to 1 where a launch cannot take it); GD_STRIP=n gives the
  * rows per strip tile (0: none).  Every form gives the same bits.  No
  * counterpart in the reference. */
 int gd_fused_phases(const gd_handle *h);
@@ -432,7 +434,7 @@ int gd_fused_phases(const gd_handle *h);
  * NULL) is a text file of earlier results keyed by the device architecture,
  * grid, member counts, precision and schemes: a cached entry is applied
  * without timing, a new result is appended.  Outputs (may be NULL): the
- * chosen form (0, 1 or 2), workgroups per member and milliseconds per
+ * chosen form (0 to 3, as GD_FUSED names them), workgroups per member and milliseconds per
  * step. */
 int gd_autotune(gd_handle *h, int32_t steps, const char *cache_path, int32_t *fused,
                 int32_t *upd_wpm, double *ms_per_step);

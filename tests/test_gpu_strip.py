@@ -1,7 +1,8 @@
 """The rows away from the polar filter in the fast and slow passes of an
 integrator call as strip tiles (GD_STRIP = rows per tile when the handle is
 created, 0: the row tiles), beside every form of the phase launches
-(GD_FUSED: 0 separate, 1 k_phase, 2 k_wphase).  All form every value by the same
+(GD_FUSED: 0 separate, 1 k_phase, 2 k_wphase, 3 k_rphase, one workgroup per
+filtered row with a wave per component).  All form every value by the same
 expressions and add every sum in the same order, so states, per-step mass,
 energy and beta must agree bit for bit; and with the oracle to the tolerance
 of the other whole-step comparisons (1e-11 after a few steps)."""
@@ -63,12 +64,12 @@ def test_strip_tiles_bitwise(gd, case, prec):
               zonal_tend_filter_cutoff_wavenumber=gd.cutoff_from_lat0(N, M, 75.0))
     print(f"strip N={N} M={M} {opts} {prec}", flush=True)
     ref = run(gd, 0, 1, N, M, dt, 3, **kw)[1]
-    for rows, form in ((4, 1), (1, 0), (7, 2), (4, 2), (0, 2), (32, 1)):
+    for rows, form in ((4, 1), (1, 0), (7, 2), (4, 2), (2, 3), (0, 2), (32, 1)):
         for x, y in zip(run(gd, rows, form, N, M, dt, 3, **kw)[1], ref):
             np.testing.assert_array_equal(x, y)
 
 
-@pytest.mark.parametrize("form", [1])
+@pytest.mark.parametrize("form", [1, 3])
 def test_strip_active_subset_and_diffusion(gd, form):
     N, M = 180, 91
     kw = dict(split_scheme="csp2", subcycles=4, use_diffusion=True, diffusion_coef=1e5, precision="mixed",
