@@ -110,6 +110,7 @@ struct gd_handle {
   RowRanges near_all, near_far;
   void *dstrip = nullptr;
   int strip_mode = -1;   // rows per strip tile: -1 by launch size
+  int fold_mode = -1;    // updates folded into the next call (use_fold): -1 by grid size
   int32_t *dstep = nullptr;
   double *ddiag = nullptr;  // [nmem][cap][3]
   int diag_cap = 512;
@@ -175,6 +176,7 @@ Args base_args(const gd_handle *h) {
   a.off_beta = h->off_beta;
   a.off_sy = h->off_sy;
   a.strip_coef = h->dstrip;
+  a.s_fold = -1;
   a.nfar_rng = 1;
   a.nfar_rows = a.far_cnt[0] = h->M;
   a.mslots = h->dmslots;
@@ -376,8 +378,38 @@ hipError_t enqueue_phase(gd_handle *h, Args a, int pass, bool in_full, bool stri
   return run(h, "phase", [&] { return launch_phase(a, h->prec, pass, in_full, h->stream); });
 }
 
-// predict_correct(dt, s0 -> s_out, pass) (dycore_mod.F90:754-792)
-hipError_t enqueue_call(gd_handle *h, double dt, int pass, int s0, int s_out, int qcon) {
+// The call before, whose state s0 + dt beta Tc -> s_out a call's phase A forms
+// itself (slot < 0: none).
+struct Pending {
+  int slot = -1, qcon = 0;
+  double dt = 0;
+};
+
+// Whether csp2's calls leave their update to the next call's phase A (GD_FOLD
+// = 0 or 1 in the environment when the handle is created overrides), which then takes the call's Tc beside its state and adds the beta partials in
+// every tile: one launch and its gap less per call, against num_lat * segments
+// more entries of 48 bytes to read per tile.  ms per step with the k_update
+// launches and without: 180x90 0.256 / 0.243, 8 members of 180x91 0.279 / 0.249,
+// 360x181 0.240 / 0.227, 405x203 0.350 / 0.336, 720x361 (1083 entries) 0.355 /
+// 0.350, two of them 0.464 / 0.442; 900x451 (1804 entries) 0.541 / 0.550,
+// 1440x721 (4326) 0.730 / 0.747.  A launch of many rounds hides the k_update
+// gap and pays for the loads: 32 of 180x91 in k_phase (2912 tiles) 0.584 /
+// 0.568, but 8 of 720x361 (8664) 1.485 / 1.546 and 64 of 360x181 (23168) 3.757 /
+// 3.850.  k_rphase, with no registers left for it, keeps k_update.
+bool use_fold(const gd_handle *h) {
+  if (h->strip_b < h->strip_a || strip_rows(h) == 0) return false;
+  const int form = strip_form(h);
+  if (form != 1 && form != 2) return false;
+  if (h->fold_mode >= 0) return h->fold_mode != 0;
+  const int64_t entries = (int64_t)h->M * ((h->N + kSeg - 1) / kSeg);
+  return entries <= 6 * kBlock && h->nact * entries <= 16 * (int64_t)h->ncu;
+}
+
+// predict_correct(dt, s0 -> s_out, pass) (dycore_mod.F90:754-792).  before: s0
+// is still to be formed from this call; leave: the update is left to the next
+// call.
+hipError_t enqueue_call(gd_handle *h, double dt, int pass, int s0, int s_out, int qcon, Pending before = Pending(),
+                        bool leave = false) {
   Args a = base_args(h);
   a.pass = pass;
   a.qcon = qcon;
@@ -395,13 +427,18 @@ hipError_t enqueue_call(gd_handle *h, double dt, int pass, int s0, int s_out, in
   }
   // first predictor: T = L(S0), S1 = S0 + dt/2 T
   a.phase = PH_A; a.s_in = s0; a.s_out = SP1;
+  a.s_fold = before.slot;
+  a.fold_qcon = before.qcon;
+  a.fold_dt = before.dt;
   if ((e = enqueue_phase(h, a, pass, s0 == SX, strip)) != hipSuccess) return e;
+  a.s_fold = -1;
   // second predictor: T = L(S1), S2 = S0 + dt/2 T, keep T
   a.phase = PH_B; a.s_in = SP1; a.s_out = SP2;
   if ((e = enqueue_phase(h, a, pass, false, strip)) != hipSuccess) return e;
   // corrector tendency T = L(S2) and the beta inner-product partials
   a.phase = PH_C; a.s_in = SP2;
   if ((e = enqueue_phase(h, a, pass, false, strip)) != hipSuccess) return e;
+  if (leave) return hipSuccess;
   a.s_out = s_out;
   return run(h, "update", [&] { return launch_update(a, h->prec, h->stream); });
 }
@@ -520,13 +557,17 @@ hipError_t enqueue_step(gd_handle *h) {
   if (c.split_scheme == GD_SPLIT_CSP2) {
     // csp2_splitting (dycore_mod.F90:671-687)
     const double fast_dt = dt / c.subcycles;
-    if ((e = enqueue_call(h, 0.5 * dt, GD_PASS_SLOW, SX, SY, c.qcon_modified)) != hipSuccess) return e;
+    const bool fold = use_fold(h);
+    Pending p;
+    if ((e = enqueue_call(h, 0.5 * dt, GD_PASS_SLOW, SX, SY, c.qcon_modified, p, fold)) != hipSuccess) return e;
+    if (fold) p = Pending{SX, c.qcon_modified, 0.5 * dt};
     int t1 = SY, t2 = SZ;
     for (int k = 0; k < c.subcycles; ++k) {
-      if ((e = enqueue_call(h, fast_dt, GD_PASS_FAST, t1, t2, c.qcon_modified)) != hipSuccess) return e;
+      if ((e = enqueue_call(h, fast_dt, GD_PASS_FAST, t1, t2, c.qcon_modified, p, fold)) != hipSuccess) return e;
+      if (fold) p = Pending{t1, c.qcon_modified, fast_dt};
       std::swap(t1, t2);
     }
-    if ((e = enqueue_call(h, 0.5 * dt, GD_PASS_SLOW, t1, t2, c.qcon_modified)) != hipSuccess) return e;
+    if ((e = enqueue_call(h, 0.5 * dt, GD_PASS_SLOW, t1, t2, c.qcon_modified, p)) != hipSuccess) return e;
     last = t2;
   } else if (c.split_scheme == GD_SPLIT_ISP) {
     if ((e = enqueue_isp_step(h, &last)) != hipSuccess) return e;
@@ -950,6 +991,8 @@ int gd_create(const gd_config *cfg, int32_t n_members, gd_handle **out) {
     h->fused_mode = env && env[0] >= '0' && env[0] <= '3' ? env[0] - '0' : -1;
     const char *bd = std::getenv("GD_STRIP");
     if (bd && bd[0]) h->strip_mode = std::max(0, std::min(std::atoi(bd), 32));
+    const char *fo = std::getenv("GD_FOLD");
+    if (fo && fo[0] >= '0' && fo[0] <= '1' && fo[1] == 0) h->fold_mode = fo[0] - '0';
     const char *nar = std::getenv("GD_UPD_NARROW");
     h->upd_narrow = nar && (nar[0] == '0' || nar[0] == '1') ? nar[0] - '0' : -1;
     // (the MFMA filter runs as its own launch between k_tend and k_filter)

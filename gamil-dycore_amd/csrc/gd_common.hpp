@@ -146,6 +146,40 @@ __device__ __forceinline__ void tend_store(const Member &mb, bool tb, int comp, 
   (tb ? mb.tb(comp) : mb.tc(comp))[o] = v;
 }
 
+// Phase A of a call may form its own state from the call before it, X' = X +
+// dt beta Tc (k_update's expression), wherever it reads it, in place of a
+// k_update launch (FOLD).  fold_step: dt beta of that call, from the member's
+// partials in k_update's order (thread tid adds entries tid, tid + kBlock, ...),
+// by every tile for itself.  `red` holds 24 doubles; ends with barriers.
+__device__ __forceinline__ double fold_step(const Args &a, const Member &mb, double *red) {
+  const int n = a.M * a.nseg, tid = ltid();
+  double q[6] = {0, 0, 0, 0, 0, 0};
+  for (int k0 = 0; k0 < n; k0 += 3 * kBlock) {
+    double2 x[3][3];
+    bool in[3];
+#pragma unroll
+    for (int u = 0; u < 3; ++u) {
+      const int k = k0 + u * kBlock + tid;
+      in[u] = k < n;
+      const int kk = in[u] ? k : 0, row = kk / a.nseg, sg = kk - row * a.nseg;
+#pragma unroll
+      for (int c = 0; c < 3; ++c) x[u][c] = *(const double2 *)(mb.part() + ((size_t)(row * 3 + c) * a.nseg + sg) * 2);
+    }
+#pragma unroll
+    for (int u = 0; u < 3; ++u)
+#pragma unroll
+      for (int c = 0; c < 3; ++c) {
+        q[2 * c] += in[u] ? x[u][c].x : 0.0;
+        q[2 * c + 1] += in[u] ? x[u][c].y : 0.0;
+      }
+  }
+  block_sum_n<6>(q, red);
+  const double ip1 = (q[0] + q[2]) + q[4];
+  const double ip2 = (q[1] + q[3]) + q[5];
+  const double beta = (a.fold_qcon && ip1 != 0.0 && ip2 != 0.0) ? ip1 / ip2 : 1.0;
+  return a.fold_dt * beta;
+}
+
 // The epilogue of one tendency value of a predict/correct phase (not
 // diffusion), split in two so a kernel can issue the load early: the value
 // phase_store needs (state s0 for the predictors, Tb for phase C) ...

@@ -147,6 +147,10 @@ struct Args {
   // (strip_rows_fill)
   int strip_a, strip_b, strip_r, strip_ngroup;
   int nstrip, strip_blk, row_blk;
+  // a phase A that applies the call before it (fold): its state s_fold, its
+  // beta from the partials with fold_qcon, its step fold_dt
+  int s_fold, fold_qcon;
+  double fold_dt;
   const void *strip_coef;
   int in_full;                 // k_diffuse: read stored u, v of s_in
   int nslots;

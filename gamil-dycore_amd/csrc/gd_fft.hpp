@@ -339,9 +339,12 @@ __device__ __forceinline__ void cplx_mid(const double2 *s, double2 *d, int L, in
 // transform path would give it.  KP: longitudes per thread (N <= KP *
 // kBlock).  tw holds tw_entries(N) entries, b0 and b1 fft_L complex points
 // each; red holds 8 doubles.  Ends with a barrier.
-template <typename CT, int KP, bool XIN>
+// FOLD: phase A's own state, weight and epilogue input alike, is s_fold + dtb
+// Tc, and the row of it is stored to s_in.
+template <typename CT, int KP, bool XIN, bool FOLD = false>
 __device__ __forceinline__ void filter_row(const Args &a, const Member &mb, const FiltRow &fr, double2 *tw,
-                                           double2 *b0, double2 *b1, double *red, bool zero = false) {
+                                           double2 *b0, double2 *b1, double *red, bool zero = false,
+                                           double dtb = 0.0) {
   const int N = a.N, P = a.pitch, L = a.fft_L, tid = threadIdx.x;
   const bool rescale = a.phase <= PH_T;
   const double sc = 1.0 / (double)L;
@@ -367,11 +370,16 @@ __device__ __forceinline__ void filter_row(const Args &a, const Member &mb, cons
     if (l < N) {
       if (!XIN) xv = xp[l];
       if (rescale) {
-        if (!zero) {
-          wv = wp[l];
+        if (FOLD) {
+          wv = pv = fld_base(mb, a.s_fold, comp, o + l) + dtb * mb.tc(comp)[o + l];
           if (gdrow) gv = wq[l];
+        } else {
+          if (!zero) {
+            wv = wp[l];
+            if (gdrow) gv = wq[l];
+          }
+          pv = phase_pre<CT>(a, mb, comp, o + l);
         }
-        pv = phase_pre<CT>(a, mb, comp, o + l);
       }
     }
     x[k] = xv;
@@ -456,6 +464,7 @@ __device__ __forceinline__ void filter_row(const Args &a, const Member &mb, cons
     const int l = tid + k * kBlock;
     if (l >= N) continue;
     const double T = rescale ? (filt ? yv[k] * s1 / s2 : x[k]) : yv[k];
+    if (FOLD) mb.st(a.s_in, comp == CDU ? FU : (comp == CDV ? FV : FGD))[o + l] = pre[k];
     if (a.phase <= PH_T) {
       phase_store<CT>(a, mb, comp, o + l, T, pre[k], fr.wrow, p[0], p[1]);
     } else if (a.phase == PH_D) {
@@ -517,9 +526,10 @@ __device__ __forceinline__ void head_sum_n(double (&v)[K], double *red) {
 // adds the products of longitudes t, t + kBlock, ... in turn (staged through
 // scr, 2 N doubles), then head_sum_n reduces those kBlock partial sums as
 // block_sum_n does, so both give the same bits.  Ends with a barrier.
-template <typename CT, int NT, int KW>
+template <typename CT, int NT, int KW, bool FOLD = false>
 __device__ __forceinline__ void filter_row_w(const Args &a, const Member &mb, const FiltRow &fr, double2 *tw,
-                                             double2 *b0, double2 *b1, double *scr, double *red, bool zero) {
+                                             double2 *b0, double2 *b1, double *scr, double *red, bool zero,
+                                             double dtb = 0.0) {
   const int N = a.N, P = a.pitch, L = a.fft_L, tid = threadIdx.x;
   const double sc = 1.0 / (double)L;
   const int comp = fr.comp;
@@ -533,11 +543,16 @@ __device__ __forceinline__ void filter_row_w(const Args &a, const Member &mb, co
     const int l = tid + k * NT;
     double wv = 0.0, gv = 0.0, pv = 0.0;
     if (l < N) {
-      if (!zero) {
-        wv = wp[l];
+      if (FOLD) {
+        wv = pv = fld_base(mb, a.s_fold, comp, o + l) + dtb * mb.tc(comp)[o + l];
         if (gdrow) gv = mb.ghs()[o + l];
+      } else {
+        if (!zero) {
+          wv = wp[l];
+          if (gdrow) gv = mb.ghs()[o + l];
+        }
+        pv = phase_pre<CT>(a, mb, comp, o + l);
       }
-      pv = phase_pre<CT>(a, mb, comp, o + l);
     }
     w[k] = wv;
     wg[k] = gv;
@@ -597,6 +612,7 @@ __device__ __forceinline__ void filter_row_w(const Args &a, const Member &mb, co
     pk[k][0] = pk[k][1] = 0.0;
     if (l < N) {
       const double T = filt ? yv[k] * s1 / s2 : x[k];
+      if (FOLD) mb.st(a.s_in, comp == CDU ? FU : (comp == CDV ? FV : FGD))[o + l] = pre[k];
       phase_store<CT>(a, mb, comp, o + l, T, pre[k], fr.wrow, pk[k][0], pk[k][1]);
     }
   }

@@ -40,7 +40,7 @@ __global__ void __launch_bounds__(kBlock) k_tend(const Args a) {
   __shared__ double red[4 * 6];
   if constexpr (STRIP) {
     if ((int)blockIdx.x >= a.row_blk) {
-      strip_block<CT, PASS, IN_FULL>(a, a.row_blk, smem);
+      strip_block<CT, PASS, IN_FULL>(a, a.row_blk, smem, red);
       return;
     }
   }

@@ -69,17 +69,17 @@ __device__ __forceinline__ void row_put(const Args &a, double *rowbuf, int l, do
 // Component CM of full row j (half row j for dv), segment by segment; the
 // loads of segment g+1 are issued before segment g is evaluated, so only the
 // first segment waits a full load round.
-template <typename CT, int PASS, bool IN_FULL, int CM>
+template <typename CT, int PASS, bool IN_FULL, int CM, bool FOLD>
 __device__ __forceinline__ void near_row(const Args &a, const Member &mb, const RowCoef &cj, int j, double *rowbuf,
-                                         unsigned char *smem, double *red) {
+                                         unsigned char *smem, double *red, double dtb) {
   const int N = a.N, tid = threadIdx.x;
   const RowNbr nb = row_nbr(a, j);
   SegLoads cur;
-  seg_load<PASS, IN_FULL>(a, mb, j, 0, min(N, kSeg), cur);
+  seg_load<PASS, IN_FULL, FOLD>(a, mb, j, 0, min(N, kSeg), cur, dtb);
   for (int g = 0; g < a.nseg; ++g) {
     const int i0 = g * kSeg, W = min(N - i0, kSeg);
     SegLoads nxt;
-    if (g + 1 < a.nseg) seg_load<PASS, IN_FULL>(a, mb, j, i0 + kSeg, min(N - i0 - kSeg, kSeg), nxt);
+    if (g + 1 < a.nseg) seg_load<PASS, IN_FULL, FOLD>(a, mb, j, i0 + kSeg, min(N - i0 - kSeg, kSeg), nxt, dtb);
     if (g) __syncthreads();  // the previous segment's stencil rows have been read
     const TendPoint pt = seg_eval<CT, PASS, IN_FULL, CM>(a, cj, nb, j, i0, W, cur, false, 0.0,
                                                          TendPoint{0, 0, 0, 0, 0, 0}, smem, red);
@@ -88,7 +88,7 @@ __device__ __forceinline__ void near_row(const Args &a, const Member &mb, const 
   }
 }
 
-template <typename CT, int PASS, bool IN_FULL, int KP>
+template <typename CT, int PASS, bool IN_FULL, int KP, bool FOLD>
 __device__ __forceinline__ void near_tile(const Args &a, const FiltRow fr, unsigned char *smem, double *red) {
   const int N = a.N, L = a.fft_L, tid = threadIdx.x;
   const Member mb = member_at(a, fr.member);
@@ -98,15 +98,16 @@ __device__ __forceinline__ void near_tile(const Args &a, const FiltRow fr, unsig
   double2 *b0 = (double2 *)(smem + phase_region0<CT>(L));
   double2 *tw = b0 + L;
   tw_to_lds(a, tw);
+  const double dtb = FOLD ? fold_step(a, mb, red) : 0.0;
   double *rowbuf = (double *)b0;
   if (fr.comp == CDU) {
-    near_row<CT, PASS, IN_FULL, TC_DU>(a, mb, cj, j, rowbuf, smem, red);
+    near_row<CT, PASS, IN_FULL, TC_DU, FOLD>(a, mb, cj, j, rowbuf, smem, red, dtb);
   } else if (fr.comp == CDV) {
-    near_row<CT, PASS, IN_FULL, TC_DV>(a, mb, cj, j, rowbuf, smem, red);
+    near_row<CT, PASS, IN_FULL, TC_DV, FOLD>(a, mb, cj, j, rowbuf, smem, red, dtb);
   } else if (PASS != 2 && (j == 0 || j == a.M - 1)) {
     // a pole row's dgd is minus the pole flux at every longitude
     // (dycore_mod.F90:572-596)
-    const double pole = pole_flux(a, mb, j, red);
+    const double pole = pole_flux<FOLD>(a, mb, j, red, dtb);
     for (int l = tid; l < N; l += kBlock) row_put(a, rowbuf, l, -pole);
   } else if (PASS == 2) {
     // the slow pass has no mass continuity term: a zero row, which a
@@ -114,11 +115,11 @@ __device__ __forceinline__ void near_tile(const Args &a, const FiltRow fr, unsig
     if (a.phase > PH_T)
       for (int l = tid; l < N; l += kBlock) row_put(a, rowbuf, l, 0.0);
   } else {
-    near_row<CT, PASS, IN_FULL, TC_DGD>(a, mb, cj, j, rowbuf, smem, red);
+    near_row<CT, PASS, IN_FULL, TC_DGD, FOLD>(a, mb, cj, j, rowbuf, smem, red, dtb);
   }
   __builtin_amdgcn_s_waitcnt(0);  // the twiddle copy has landed
   __syncthreads();  // row and twiddles published; the stencil rows are free for b1
-  filter_row<CT, KP, true>(a, mb, fr, tw, b0, b1, red, PASS == 2 && fr.comp == CDGD && a.phase <= PH_T);
+  filter_row<CT, KP, true, FOLD>(a, mb, fr, tw, b0, b1, red, PASS == 2 && fr.comp == CDGD && a.phase <= PH_T, dtb);
 }
 
 // Four longitudes per thread (rows up to 1024): five waves per SIMD (at most
@@ -131,7 +132,7 @@ __device__ __forceinline__ void near_tile(const Args &a, const FiltRow fr, unsig
 template <int KP, bool STRIP>
 constexpr int phase_waves() { return KP == 4 ? (STRIP ? 4 : 5) : 3; }
 
-template <typename CT, int PASS, bool IN_FULL, int KP, bool STRIP>
+template <typename CT, int PASS, bool IN_FULL, int KP, bool STRIP, bool FOLD = false>
 __global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(phase_waves<KP, STRIP>(), 8)))
 k_phase(const Args a) {
   extern __shared__ __align__(16) unsigned char smem[];
@@ -144,12 +145,12 @@ k_phase(const Args a) {
     const int t = (b % kXcd) * (a.nnear_pad / kXcd) + b / kXcd;
     // (the row descriptor is copied: a reference into global memory would be
     // reloaded after every store of the epilogue)
-    if (t < a.nnear) near_tile<CT, PASS, IN_FULL, KP>(a, a.frows[t], smem, red);
+    if (t < a.nnear) near_tile<CT, PASS, IN_FULL, KP, FOLD>(a, a.frows[t], smem, red);
     return;
   }
   if constexpr (STRIP) {
     if (b >= a.nnear_pad + a.row_blk) {
-      strip_block<CT, PASS, IN_FULL>(a, a.nnear_pad + a.row_blk, smem);
+      strip_block<CT, PASS, IN_FULL, 1, FOLD>(a, a.nnear_pad + a.row_blk, smem, red);
       return;
     }
   }
@@ -158,7 +159,7 @@ k_phase(const Args a) {
   const int bb = b - a.nnear_pad, per = a.row_blk / kXcd;
   const int t = (bb % kXcd) * per + bb / kXcd;
   if (t >= a.ntiles) return;
-  tend_tile<CT, PASS, IN_FULL, true>(a, t, smem, red);
+  tend_tile<CT, PASS, IN_FULL, true, FOLD>(a, t, smem, red);
 }
 
 // ---------------------------------------------------------------------------
@@ -206,20 +207,20 @@ __host__ __device__ inline size_t wphase_lds(int N, int L) {
 // segment's loads issued before the current one is evaluated).  A tile with
 // no segment left in a round evaluates an empty one (W = 0: its loads stay
 // inside the row, nothing is written) to take the round's barriers.
-template <typename CT, int PASS, bool IN_FULL, int CM>
+template <typename CT, int PASS, bool IN_FULL, int CM, bool FOLD>
 __device__ __forceinline__ void wnear_row(const Args &a, const Member &mb, const RowCoef &cj, int j, int s,
-                                          double *rowbuf, unsigned char *st, double *red) {
+                                          double *rowbuf, unsigned char *st, double *red, double dtb) {
   const int N = a.N, nseg = a.nseg, tid = ltid();
   const int rounds = (nseg + kWTiles - 1) / kWTiles;
   const RowNbr nb = row_nbr(a, j);
   auto seg_i0 = [&](int g) { return g < nseg ? g * kSeg : 0; };
   auto seg_w = [&](int g) { return g < nseg ? min(N - g * kSeg, kSeg) : 0; };
   SegLoads cur;
-  seg_load<PASS, IN_FULL>(a, mb, j, seg_i0(s), seg_w(s), cur);
+  seg_load<PASS, IN_FULL, FOLD>(a, mb, j, seg_i0(s), seg_w(s), cur, dtb);
   for (int k = 0; k < rounds; ++k) {
     const int g = k * kWTiles + s, gn = g + kWTiles;
     SegLoads nxt;
-    if (k + 1 < rounds) seg_load<PASS, IN_FULL>(a, mb, j, seg_i0(gn), seg_w(gn), nxt);
+    if (k + 1 < rounds) seg_load<PASS, IN_FULL, FOLD>(a, mb, j, seg_i0(gn), seg_w(gn), nxt, dtb);
     if (k) __syncthreads();  // the previous round's stencil rows have been read
     const int i0 = seg_i0(g), W = seg_w(g);
     const TendPoint pt = seg_eval<CT, PASS, IN_FULL, CM>(a, cj, nb, j, i0, W, cur, false, 0.0,
@@ -229,7 +230,7 @@ __device__ __forceinline__ void wnear_row(const Args &a, const Member &mb, const
   }
 }
 
-template <typename CT, int PASS, bool IN_FULL, int KW>
+template <typename CT, int PASS, bool IN_FULL, int KW, bool FOLD>
 __device__ __forceinline__ void wnear_tile(const Args &a, const FiltRow fr, unsigned char *smem, double *red) {
   constexpr int NT = kWTiles * kBlock;
   const int N = a.N, L = a.fft_L, s = threadIdx.x / kBlock;
@@ -244,29 +245,30 @@ __device__ __forceinline__ void wnear_tile(const Args &a, const FiltRow fr, unsi
   double *rowbuf = (double *)b0;
   unsigned char *st = smem + s * R;
   double *rd = red + s * 4 * 6;
+  const double dtb = FOLD ? fold_step(a, mb, rd) : 0.0;
   if (fr.comp == CDU) {
-    wnear_row<CT, PASS, IN_FULL, TC_DU>(a, mb, cj, j, s, rowbuf, st, rd);
+    wnear_row<CT, PASS, IN_FULL, TC_DU, FOLD>(a, mb, cj, j, s, rowbuf, st, rd, dtb);
   } else if (fr.comp == CDV) {
-    wnear_row<CT, PASS, IN_FULL, TC_DV>(a, mb, cj, j, s, rowbuf, st, rd);
+    wnear_row<CT, PASS, IN_FULL, TC_DV, FOLD>(a, mb, cj, j, s, rowbuf, st, rd, dtb);
   } else if (PASS != 2 && (j == 0 || j == a.M - 1)) {
     // a pole row's dgd is minus the pole flux at every longitude; each tile
     // forms the same ring sum (dycore_mod.F90:572-596)
-    const double pole = pole_flux(a, mb, j, rd);
+    const double pole = pole_flux<FOLD>(a, mb, j, rd, dtb);
     for (int l = threadIdx.x; l < N; l += NT) row_put(a, rowbuf, l, -pole);
   } else if (PASS != 2) {
-    wnear_row<CT, PASS, IN_FULL, TC_DGD>(a, mb, cj, j, s, rowbuf, st, rd);
+    wnear_row<CT, PASS, IN_FULL, TC_DGD, FOLD>(a, mb, cj, j, s, rowbuf, st, rd, dtb);
   }
   // (the slow pass has no mass continuity term: its dgd rows are zero rows,
   // which filter_row_w leaves unfiltered without reading b0)
   __builtin_amdgcn_s_waitcnt(0);  // the twiddle copy has landed
   __syncthreads();  // row and twiddles published; the stencil rows are free
-  filter_row_w<CT, NT, KW>(a, mb, fr, tw, b0, b1, (double *)(smem + R), red, PASS == 2 && fr.comp == CDGD);
+  filter_row_w<CT, NT, KW, FOLD>(a, mb, fr, tw, b0, b1, (double *)(smem + R), red, PASS == 2 && fr.comp == CDGD, dtb);
 }
 
 // Two workgroups per CU (16 of the 20 waves that 96 VGPRs allow).  KW:
 // longitudes per thread in the filter (1 up to 512 longitudes, 2 up to 1024).
 // STRIP: with strip tiles (four waves per SIMD, as k_phase).
-template <typename CT, int PASS, bool IN_FULL, int KW, bool STRIP>
+template <typename CT, int PASS, bool IN_FULL, int KW, bool STRIP, bool FOLD = false>
 __global__ void __launch_bounds__(kWTiles * kBlock) __attribute__((amdgpu_waves_per_eu(STRIP ? 4 : 5, 8)))
 k_wphase(const Args a) {
   extern __shared__ __align__(16) unsigned char smem[];
@@ -274,12 +276,12 @@ k_wphase(const Args a) {
   const int b = blockIdx.x;
   if (b < a.nnear_pad) {
     const int t = (b % kXcd) * (a.nnear_pad / kXcd) + b / kXcd;
-    if (t < a.nnear) wnear_tile<CT, PASS, IN_FULL, KW>(a, a.frows[t], smem, red);
+    if (t < a.nnear) wnear_tile<CT, PASS, IN_FULL, KW, FOLD>(a, a.frows[t], smem, red);
     return;
   }
   if constexpr (STRIP) {
     if (b >= a.nnear_pad + a.row_blk) {
-      strip_block<CT, PASS, IN_FULL, kWTiles>(a, a.nnear_pad + a.row_blk, smem);
+      strip_block<CT, PASS, IN_FULL, kWTiles, FOLD>(a, a.nnear_pad + a.row_blk, smem, red);
       return;
     }
   }
@@ -298,8 +300,8 @@ k_wphase(const Args a) {
   }
   const int s = threadIdx.x / kBlock;
   const bool live = t0 + s < a.ntiles;
-  tend_tile<CT, PASS, IN_FULL, true>(a, live ? t0 + s : a.ntiles - 1, smem + s * wphase_region<CT>(a.fft_L),
-                                     red + s * 4 * 6, bar2, live);
+  tend_tile<CT, PASS, IN_FULL, true, FOLD>(a, live ? t0 + s : a.ntiles - 1, smem + s * wphase_region<CT>(a.fft_L),
+                                           red + s * 4 * 6, bar2, live);
 }
 
 // ---------------------------------------------------------------------------
@@ -376,7 +378,7 @@ k_rphase(const Args a) {
     return;
   }
   if (b >= a.nnear_pad + a.row_blk) {
-    strip_block<CT, PASS, IN_FULL>(a, a.nnear_pad + a.row_blk, smem);
+    strip_block<CT, PASS, IN_FULL>(a, a.nnear_pad + a.row_blk, smem, red);
     return;
   }
   const int bb = b - a.nnear_pad, t = (bb % kXcd) * (a.row_blk / kXcd) + bb / kXcd;
@@ -484,7 +486,13 @@ static hipError_t launch_phase_k(Args a, int pass, bool in_full, hipStream_t s) 
   dim3 g(a.nnear_pad + a.row_blk + a.strip_blk), b(kBlock);
   const size_t lds = phase_lds_t<CT>(a.N, a.fft_L);
 #define GD_PH(P, F, S) hipLaunchKernelGGL((k_phase<CT, P, F, KP, S>), g, b, lds, s, a)
-  if (a.nstrip > 0) {
+  if (a.s_fold >= 0) {
+    if (pass == 0 || in_full || a.nstrip <= 0) return hipErrorInvalidValue;
+    if (pass == 1)
+      hipLaunchKernelGGL((k_phase<CT, 1, false, KP, true, true>), g, b, lds, s, a);
+    else
+      hipLaunchKernelGGL((k_phase<CT, 2, false, KP, true, true>), g, b, lds, s, a);
+  } else if (a.nstrip > 0) {
     if (pass == 0) return hipErrorInvalidValue;
     if (pass == 1) { if (in_full) GD_PH(1, true, true); else GD_PH(1, false, true); }
     else { if (in_full) GD_PH(2, true, true); else GD_PH(2, false, true); }
@@ -549,7 +557,13 @@ static hipError_t launch_wphase_k(Args a, int pass, bool in_full, hipStream_t s)
   dim3 g(a.nnear_pad + a.row_blk + a.strip_blk), b(kWTiles * kBlock);
   const size_t lds = wphase_lds<CT>(a.N, a.fft_L);
 #define GD_PH(P, F, S) hipLaunchKernelGGL((k_wphase<CT, P, F, KW, S>), g, b, lds, s, a)
-  if (a.nstrip > 0) {
+  if (a.s_fold >= 0) {
+    if (pass == 0 || in_full || a.nstrip <= 0) return hipErrorInvalidValue;
+    if (pass == 1)
+      hipLaunchKernelGGL((k_wphase<CT, 1, false, KW, true, true>), g, b, lds, s, a);
+    else
+      hipLaunchKernelGGL((k_wphase<CT, 2, false, KW, true, true>), g, b, lds, s, a);
+  } else if (a.nstrip > 0) {
     if (pass == 0) return hipErrorInvalidValue;
     if (pass == 1) { if (in_full) GD_PH(1, true, true); else GD_PH(1, false, true); }
     else { if (in_full) GD_PH(2, true, true); else GD_PH(2, false, true); }
@@ -579,7 +593,8 @@ static hipError_t configure_wphase_k(int max_lds) {
                        (const void *)k_wphase<CT, 1, true, KW, false>, (const void *)k_wphase<CT, 1, false, KW, false>,
                        (const void *)k_wphase<CT, 2, true, KW, false>, (const void *)k_wphase<CT, 2, false, KW, false>,
                        (const void *)k_wphase<CT, 1, true, KW, true>,  (const void *)k_wphase<CT, 1, false, KW, true>,
-                       (const void *)k_wphase<CT, 2, true, KW, true>,  (const void *)k_wphase<CT, 2, false, KW, true>};
+                       (const void *)k_wphase<CT, 2, true, KW, true>,  (const void *)k_wphase<CT, 2, false, KW, true>,
+                       (const void *)k_wphase<CT, 1, false, KW, true, true>, (const void *)k_wphase<CT, 2, false, KW, true, true>};
   for (const void *f : fns) {
     hipError_t e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, max_lds);
     if (e != hipSuccess) return e;
@@ -593,7 +608,8 @@ static hipError_t configure_phase_k(int max_lds) {
                        (const void *)k_phase<CT, 1, true, KP, false>, (const void *)k_phase<CT, 1, false, KP, false>,
                        (const void *)k_phase<CT, 2, true, KP, false>, (const void *)k_phase<CT, 2, false, KP, false>,
                        (const void *)k_phase<CT, 1, true, KP, true>,  (const void *)k_phase<CT, 1, false, KP, true>,
-                       (const void *)k_phase<CT, 2, true, KP, true>,  (const void *)k_phase<CT, 2, false, KP, true>};
+                       (const void *)k_phase<CT, 2, true, KP, true>,  (const void *)k_phase<CT, 2, false, KP, true>,
+                       (const void *)k_phase<CT, 1, false, KP, true, true>, (const void *)k_phase<CT, 2, false, KP, true, true>};
   for (const void *f : fns) {
     hipError_t e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, max_lds);
     if (e != hipSuccess) return e;

@@ -98,7 +98,7 @@ __device__ __forceinline__ void st(double *base, unsigned off, double v) { *(dou
 // east or west; Fyp, Wp: of the row before.
 template <typename CT>
 struct FastRow {
-  double gd, gde, h, he, G, Ge, V, Fx, Fxw, Fyp;
+  double gd, gde, h, he, G, Ge, U, V, Fx, Fxw, Fyp;
   CT t, Q, Qw, W, Wp;  // f + c u, (f + c u) U, V + V(i+1)
 };
 
@@ -120,8 +120,10 @@ __host__ __device__ constexpr size_t strip_lds_bytes(int rows) { return (size_t)
 
 // Phase a.phase (PH_A, PH_B or PH_C) of tile t = (member, group of a.strip_r
 // rows, segment), segment fastest.  live = false: no stores (a spare tile).
-template <typename CT, int PASS, bool FULL>
-__device__ __forceinline__ void strip_tile(const Args &a, int t, bool live, unsigned char *smem) {
+// FOLD: phase A's state is s_fold + dt beta Tc, formed where a row is loaded,
+// and stored to s_in.  `red`: 24 doubles.
+template <typename CT, int PASS, bool FULL, bool FOLD>
+__device__ __forceinline__ void strip_tile(const Args &a, int t, bool live, unsigned char *smem, double *red) {
   const int N = a.N, nseg = a.nseg, tid = ltid(), lane = threadIdx.x & 63, wv = (threadIdx.x >> 6) & 3;
   const int seg = t % nseg, q = t / nseg, grp = q % a.strip_ngroup, m = q / a.strip_ngroup;
   const Member mb = member_at(a, a.m0 + m);
@@ -129,6 +131,7 @@ __device__ __forceinline__ void strip_tile(const Args &a, int t, bool live, unsi
   const int i0 = seg * kSeg, W = min(N - i0, kSeg);
   const bool first = lane == 0, last = lane == 63, pc = a.phase == PH_C;
   double *sums = (double *)smem;
+  const double dtb = FOLD ? fold_step(a, mb, red) : 0.0;
   // (a wave past the segment's end has nothing to do but its zero sums)
   const bool busy = __builtin_amdgcn_readfirstlane(wv * 64) < W;
   if (busy) {
@@ -141,7 +144,13 @@ __device__ __forceinline__ void strip_tile(const Args &a, int t, bool live, unsi
     // is inside the row)
     const int ic = i0 + min(tid, W + 1);
     const unsigned c0 = wrap(ic), cx = wrap(ic + (last ? 1 : (first ? -1 : 0)));
-    const double *gd = mb.st(a.s_in, FGD), *Ug = mb.st(a.s_in, FU), *Vg = mb.st(a.s_in, FV), *hg = mb.ghs();
+    const int si = FOLD ? a.s_fold : a.s_in;
+    const double *gd = mb.st(si, FGD), *Ug = mb.st(si, FU), *Vg = mb.st(si, FV), *hg = mb.ghs();
+    const double *tg = mb.tc(CDGD), *tu = mb.tc(CDU), *tv = mb.tc(CDV);
+    auto in = [&](const double *f, const double *tc, unsigned o) {
+      if constexpr (FOLD) return ld(f, o) + dtb * ld(tc, o);
+      return ld(f, o);
+    };
     const double *ug = mb.st(a.s_in, Fu), *vg = mb.st(a.s_in, Fv);
     // what the epilogue reads at the point (S0, or Tb in phase C) and where it
     // writes
@@ -164,6 +173,11 @@ __device__ __forceinline__ void strip_tile(const Args &a, int t, bool live, unsi
           pq[4] += xg * dg * c.fcos;
           pq[5] += dg * dg * c.fcos;
         } else {
+          if (FOLD) {
+            st(mb.st(a.s_in, FU), o, xu);
+            st(mb.st(a.s_in, FV), o, xv);
+            st(mb.st(a.s_in, FGD), o, xg);
+          }
           st(ou, o, xu + a.hdt * du);
           st(ov, o, xv + a.hdt * dv);
           st(og, o, xg + a.hdt * dg);
@@ -182,16 +196,16 @@ __device__ __forceinline__ void strip_tile(const Args &a, int t, bool live, unsi
       };
       // x: U of the western neighbour for lane 0, V of the eastern for lane 63
       const unsigned cuv = cx;
-      const double *xg_ = first ? Ug : Vg;
+      const double *xg_ = first ? Ug : Vg, *xt_ = first ? tu : tv;
       auto load = [&](int row) {
         const unsigned o = (unsigned)row * P8;
         Ld l;
-        l.g = ld(gd, o + c0);
-        l.U = ld(Ug, o + c0);
-        l.V = ld(Vg, o + c0);
+        l.g = in(gd, tg, o + c0);
+        l.U = in(Ug, tu, o + c0);
+        l.V = in(Vg, tv, o + c0);
         l.h = ld(hg, o + c0);
-        l.gx = ld(gd, o + cx);
-        l.x = ld(xg_, o + cuv);
+        l.gx = in(gd, tg, o + cx);
+        l.x = in(xg_, xt_, o + cuv);
         l.hx = ld(hg, o + cx);
         l.u = FULL ? ld(ug, o + c0) : 0.0;
         l.ux = FULL ? ld(ug, o + cx) : 0.0;
@@ -201,6 +215,7 @@ __device__ __forceinline__ void strip_tile(const Args &a, int t, bool live, unsi
         FastRow<CT> x;
         x.gd = l.g;
         x.h = l.h;
+        x.U = l.U;
         x.V = l.V;
         x.G = sqrt(l.g);
         const double Gx = sqrt(l.gx);
@@ -233,7 +248,7 @@ __device__ __forceinline__ void strip_tile(const Args &a, int t, bool live, unsi
       }
       for (int j = r0; j <= r1; ++j) {
         const unsigned o = (unsigned)j * P8 + c0;
-        const double xu = ld(pu, o), xv = ld(pv, o), xg = ld(pg, o);
+        const double xu = FOLD ? s.U : ld(pu, o), xv = FOLD ? s.V : ld(pv, o), xg = FOLD ? s.gd : ld(pg, o);
         const Ld l = l2;
         l2 = load(min(j + 2, r1 + 1));
         const StripRow<CT> cn = strip_row<CT>(a, j + 1);
@@ -264,13 +279,13 @@ __device__ __forceinline__ void strip_tile(const Args &a, int t, bool live, unsi
       auto load = [&](int row) {
         const unsigned o = (unsigned)row * P8, on = o + P8;
         Ld l;
-        l.g = ld(gd, on + c0);
-        l.gx = ld(gd, on + cx);
-        l.gy = FULL ? 0.0 : ld(gd, on + cy);
-        l.U = ld(Ug, o + c0);
-        l.V = ld(Vg, o + c0);
-        l.Ux = ld(Ug, o + cx);
-        l.Vx = ld(Vg, o + cx);
+        l.g = in(gd, tg, on + c0);
+        l.gx = in(gd, tg, on + cx);
+        l.gy = FULL ? 0.0 : in(gd, tg, on + cy);
+        l.U = in(Ug, tu, o + c0);
+        l.V = in(Vg, tv, o + c0);
+        l.Ux = in(Ug, tu, o + cx);
+        l.Vx = in(Vg, tv, o + cx);
         l.u = FULL ? ld(ug, o + c0) : 0.0;
         l.v = FULL ? ld(vg, o + c0) : 0.0;
         l.ux = FULL ? ld(ug, o + cx) : 0.0;
@@ -280,9 +295,9 @@ __device__ __forceinline__ void strip_tile(const Args &a, int t, bool live, unsi
       const unsigned op = (unsigned)(r0 - 1) * P8;
       double G = 0, Gx = 0, Gy = 0;  // sqrt gd of the row to come
       if (!FULL) {
-        G = sqrt(ld(gd, op + c0));
-        Gx = sqrt(ld(gd, op + cx));
-        Gy = sqrt(ld(gd, op + cy));
+        G = sqrt(in(gd, tg, op + c0));
+        Gx = sqrt(in(gd, tg, op + cx));
+        Gy = sqrt(in(gd, tg, op + cy));
       }
       auto row_from = [&](const Ld &l, const StripRow<CT> &c) {
         CT u, v, ux, vx;
@@ -329,7 +344,8 @@ __device__ __forceinline__ void strip_tile(const Args &a, int t, bool live, unsi
       CT Up = p.U, Vp = p.V, Yp = p.Y, Zp = p.Z;
       for (int j = r0; j <= r1; ++j) {
         const unsigned o = (unsigned)j * P8 + c0;
-        const double xu = ld(pu, o), xv = ld(pv, o), xg = ld(pg, o);
+        const double xu = FOLD ? in(Ug, tu, o) : ld(pu, o), xv = FOLD ? in(Vg, tv, o) : ld(pv, o);
+        const double xg = FOLD ? in(gd, tg, o) : ld(pg, o);
         const Ld l = l0;
         l0 = load(min(j + 2, r1 + 1));
         const StripRow<CT> cn = strip_row<CT>(a, j + 1);
@@ -366,14 +382,14 @@ __device__ __forceinline__ void strip_tile(const Args &a, int t, bool live, unsi
 // in each, every XCD a contiguous run (base and strip_blk are multiples of
 // kXcd).  A spare tile past the last does the last one's work and barriers
 // without its stores.
-template <typename CT, int PASS, bool FULL, int TILES = 1>
-__device__ __forceinline__ void strip_block(const Args &a, int base, unsigned char *smem) {
+template <typename CT, int PASS, bool FULL, int TILES = 1, bool FOLD = false>
+__device__ __forceinline__ void strip_block(const Args &a, int base, unsigned char *smem, double *red) {
   const int b = (int)blockIdx.x - base;
   const int t0 = ((b % kXcd) * (a.strip_blk / kXcd) + b / kXcd) * TILES;
   if (t0 >= a.nstrip) return;
   const int s = TILES > 1 ? (int)threadIdx.x / kBlock : 0, t = t0 + s;
-  strip_tile<CT, PASS, FULL>(a, __builtin_amdgcn_readfirstlane(min(t, a.nstrip - 1)), t < a.nstrip,
-                             smem + s * strip_lds_bytes(a.strip_r));
+  strip_tile<CT, PASS, FULL, FOLD>(a, __builtin_amdgcn_readfirstlane(min(t, a.nstrip - 1)), t < a.nstrip,
+                                   smem + s * strip_lds_bytes(a.strip_r), red + s * 4 * 6);
 }
 
 }  // namespace gd

@@ -41,10 +41,12 @@ constexpr int TC_DU = 1, TC_DV = 2, TC_DGD = 4, TC_RING = 8, TC_ALL = 15;
 // tid + kBlock, ... in that order.  The loads go in blocks of four, each
 // issued without a condition: past N a lane reads the ghost rows (gd 1,
 // V 0), whose term (1 + 1) * 0 = +0 leaves the sum as it is.
-__device__ __forceinline__ double ring_part(const Args &a, const Member &mb, int j) {
+template <bool FOLD = false>
+__device__ __forceinline__ double ring_part(const Args &a, const Member &mb, int j, double dtb = 0.0) {
   const int N = a.N, M = a.M, P = a.pitch, tid = ltid();
-  const double *gd = mb.st(a.s_in, FGD);
-  const double *Vg = mb.st(a.s_in, FV);
+  const int si = FOLD ? a.s_fold : a.s_in;
+  const double *gd = mb.st(si, FGD);
+  const double *Vg = mb.st(si, FV);
   const double *one = a.ghost, *zero = a.ghost + P;
   const int jn = j == 0 ? 1 : M - 2, hr = j == 0 ? 0 : M - 2;
   double pacc = 0.0;
@@ -58,6 +60,11 @@ __device__ __forceinline__ double ring_part(const Args &a, const Member &mb, int
       g0[k] = (in ? gd + (size_t)j * P : one)[qc];
       g1[k] = (in ? gd + (size_t)jn * P : one)[qc];
       v[k] = (in ? Vg + (size_t)hr * P : zero)[qc];
+      if (FOLD) {
+        g0[k] = g0[k] + dtb * (in ? mb.tc(CDGD) + (size_t)j * P : zero)[qc];
+        g1[k] = g1[k] + dtb * (in ? mb.tc(CDGD) + (size_t)jn * P : zero)[qc];
+        v[k] = v[k] + dtb * (in ? mb.tc(CDV) + (size_t)hr * P : zero)[qc];
+      }
     }
 #pragma unroll
     for (int k = 0; k < 4; ++k) pacc += (sqrt(g0[k]) + sqrt(g1[k])) * v[k];
@@ -65,9 +72,10 @@ __device__ __forceinline__ double ring_part(const Args &a, const Member &mb, int
   return pacc;
 }
 
-__device__ __forceinline__ double pole_flux(const Args &a, const Member &mb, int j, double *red) {
+template <bool FOLD = false>
+__device__ __forceinline__ double pole_flux(const Args &a, const Member &mb, int j, double *red, double dtb = 0.0) {
   const int N = a.N, M = a.M;
-  double sum = block_sum(ring_part(a, mb, j), red);
+  double sum = block_sum(ring_part<FOLD>(a, mb, j, dtb), red);
   if (j == M - 1) sum = -sum;
   return sum * 2.0 / N / kRadius / a.dlat;
 }
@@ -80,12 +88,15 @@ struct SegLoads {
   double g_i, g_ip, h_i, h_ip, g_n, h_n;
 };
 
-template <int PASS, bool IN_FULL>
-__device__ __forceinline__ void seg_load(const Args &a, const Member &mb, int j, int i0, int W, SegLoads &L) {
+// FOLD: the state is s_fold + dtb Tc (fold_step).
+template <int PASS, bool IN_FULL, bool FOLD = false>
+__device__ __forceinline__ void seg_load(const Args &a, const Member &mb, int j, int i0, int W, SegLoads &L,
+                                         double dtb = 0.0) {
   const int N = a.N, M = a.M, P = a.pitch, tid = ltid();
-  const double *gd = mb.st(a.s_in, FGD);
-  const double *Ug = mb.st(a.s_in, FU);
-  const double *Vg = mb.st(a.s_in, FV);
+  const int si = FOLD ? a.s_fold : a.s_in;
+  const double *gd = mb.st(si, FGD);
+  const double *Ug = mb.st(si, FU);
+  const double *Vg = mb.st(si, FV);
   const double *ghs = mb.ghs();
   auto wrap = [N](int i) { return i < 0 ? i + N : (i >= N ? i - N : i); };
   const int lcol = tid < W ? i0 + tid : (tid == W ? i0 - 1 : i0 + W);
@@ -114,6 +125,25 @@ __device__ __forceinline__ void seg_load(const Args &a, const Member &mb, int j,
     L.lU[r] = (in(row, M - 1) ? Ug + (size_t)row * P : zero)[p];
     L.lV[r] = (in(row, M - 2) ? Vg + (size_t)row * P : zero)[p];
     L.lfv[r] = IN_FULL ? (in(row, M - 2) ? mb.st(a.s_in, Fv) + (size_t)row * P : zero)[p] : 0.0;
+  }
+  if constexpr (FOLD) {
+    const double *tg = mb.tc(CDGD), *tu = mb.tc(CDU), *tv = mb.tc(CDV);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int row = j - 1 + r;
+      L.lg[r] = L.lg[r] + dtb * (in(row, M - 1) ? tg + (size_t)row * P : zero)[p];
+    }
+#pragma unroll
+    for (int r = 0; r < 2; ++r) {
+      const int row = j + r;
+      L.lgn[r] = L.lgn[r] + dtb * (in(row, M - 1) ? tg + (size_t)row * P : zero)[pn];
+    }
+#pragma unroll
+    for (int r = 0; r < 3; ++r) {
+      const int row = j - 1 + r;
+      L.lU[r] = L.lU[r] + dtb * (in(row, M - 1) ? tu + (size_t)row * P : zero)[p];
+      L.lV[r] = L.lV[r] + dtb * (in(row, M - 2) ? tv + (size_t)row * P : zero)[p];
+    }
   }
   // the own point's geopotential: gd at (j, i), (j, i+1), (j+1, i) is the
   // column load already made (lg[1], lgn[0], lg[2]); only ghs is loaded
@@ -353,23 +383,28 @@ __device__ __forceinline__ TendPoint seg_eval(const Args &a, const RowCoef &cj, 
 // barrier (neighbour rows to LDS, the point's own rows, geopotential terms
 // and epilogue inputs to registers).  CM selects the components.  smem holds
 // tend_stencil_bytes<CT>() bytes, red 24 doubles.
-template <typename CT, int PASS, bool IN_FULL, int CM = TC_ALL>
+template <typename CT, int PASS, bool IN_FULL, int CM = TC_ALL, bool FOLD = false>
 __device__ __forceinline__ TendPoint tend_segment(const Args &a, const Member &mb, const RowCoef &cj, int j,
                                                   int i0, int W, bool stg_u, bool stg_v, bool stg_g,
-                                                  unsigned char *smem, double *red, bool bar2 = false) {
+                                                  unsigned char *smem, double *red, bool bar2 = false,
+                                                  double dtb = 0.0) {
   const int M = a.M, P = a.pitch, tid = ltid();
   // pole mass flux sums over the whole ring (dycore_mod.F90:572-596); every
   // segment of a pole row forms the same sum in the same order (ring_part,
   // as pole_flux).  Pole tiles finish these loads before issuing the halo
   // loads, so the two sets of registers are never live together.
   const bool pole_row = (CM & TC_RING) != 0 && PASS != 2 && (j == 0 || j == M - 1);
-  const double pacc = pole_row ? ring_part(a, mb, j) : 0.0;
+  const double pacc = pole_row ? ring_part<FOLD>(a, mb, j, dtb) : 0.0;
   const RowNbr nb = row_nbr(a, j);
   SegLoads L;
-  seg_load<PASS, IN_FULL>(a, mb, j, i0, W, L);
+  seg_load<PASS, IN_FULL, FOLD>(a, mb, j, i0, W, L, dtb);
   // the epilogue inputs of the own point
   TendPoint out{0, 0, 0, 0, 0, 0};
-  if (tid < W) {
+  if (FOLD) {
+    out.pre_u = L.lU[1];
+    out.pre_v = L.lV[1];
+    out.pre_g = L.lg[1];
+  } else if (tid < W) {
     const size_t o = (size_t)j * P + i0 + tid;
     if (!stg_u) out.pre_u = phase_pre<CT>(a, mb, CDU, o);
     if (!stg_v && j <= M - 2) out.pre_v = phase_pre<CT>(a, mb, CDV, o);
@@ -400,7 +435,7 @@ __device__ __forceinline__ int far_tile_row(const Args &a, int t) {
 
 // bar2: see seg_eval.  live = false: the tile's work and barriers without
 // its stores (a workgroup's spare tile past the last one).
-template <typename CT, int PASS, bool IN_FULL, bool FUSED>
+template <typename CT, int PASS, bool IN_FULL, bool FUSED, bool FOLD = false>
 __device__ __forceinline__ void tend_tile(const Args &a, int t, unsigned char *smem, double *red, bool bar2 = false,
                                           bool live = true) {
   const int M = a.M, P = a.pitch, nseg = a.nseg, tid = ltid();
@@ -415,12 +450,19 @@ __device__ __forceinline__ void tend_tile(const Args &a, int t, unsigned char *s
   const int st_v = has_v ? cj.stage[CDV] : -1;
   const int st_g = cj.stage[CDGD];
   const int i0 = g * kSeg, W = min(a.N - i0, kSeg);
-  const TendPoint pt = tend_segment<CT, PASS, IN_FULL>(a, mb, cj, j, i0, W, st_u >= 0, st_v >= 0, st_g >= 0,
-                                                       smem, red, bar2);
+  const double dtb = FOLD ? fold_step(a, mb, red) : 0.0;
+  const TendPoint pt = tend_segment<CT, PASS, IN_FULL, TC_ALL, FOLD>(a, mb, cj, j, i0, W, st_u >= 0, st_v >= 0,
+                                                                     st_g >= 0, smem, red, bar2, dtb);
   double p1[3] = {0, 0, 0}, p2[3] = {0, 0, 0};
   if (live && tid < W) {
     const int i = i0 + tid;
     const size_t o = (size_t)j * P + i;
+    if (FOLD) {
+      // the state the fold forms is stored for the phases to come
+      if (st_u < 0) mb.st(a.s_in, FU)[o] = pt.pre_u;
+      if (st_v < 0 && has_v) mb.st(a.s_in, FV)[o] = pt.pre_v;
+      if (st_g < 0) mb.st(a.s_in, FGD)[o] = pt.pre_g;
+    }
     // (pole rows: du = 0 goes through the epilogue like any other value)
     if (st_u < 0)
       phase_store<CT>(a, mb, CDU, o, pt.du, pt.pre_u, cj.fcos, p1[0], p2[0]);
