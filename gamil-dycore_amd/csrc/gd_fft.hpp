@@ -358,7 +358,8 @@ __device__ __forceinline__ void filter_row(const Args &a, const Member &mb, cons
   // issued together; gd + ghs is added after the forward transform, when
   // the loads have long arrived
   double *const sxb = a.sx_ext ? a.sx_ext : mb.sx();
-  const double *xp = sxb + (size_t)fr.slot * P;
+  const size_t xo = a.sx_ext && a.sx_ld ? (size_t)fr.row * a.sx_ld : (size_t)fr.slot * P;
+  const double *xp = sxb + xo;
   const double *wp = mb.st(a.s_in, comp == CDU ? FU : (comp == CDV ? FV : FGD)) + o;
   const bool gdrow = comp == CDGD;
   const double *wq = mb.ghs() + o;
@@ -482,8 +483,8 @@ __device__ __forceinline__ void filter_row(const Args &a, const Member &mb, cons
                                    : mb.st(a.s_in, FV)[o + l] * 2.0 / (sqrt(sgd[o + l]) + sqrt(sgd[o + P + l]));
         mb.st(SX, Fv)[o + l] = v + a.kdiff * T;
       }
-    } else {  // PH_P: projection only, back into the staging row
-      sxb[(size_t)fr.slot * P + l] = T;
+    } else {  // PH_P: projection only, back into its row
+      sxb[xo + l] = T;
     }
   }
   if (a.phase == PH_C) {

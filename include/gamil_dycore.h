@@ -173,13 +173,15 @@ int gd_filter_rows(gd_handle *h, int32_t half, double *x, int64_t ld);
  * allocate device memory (code under HIP graph capture, tight serving loops,
  * harnesses that forbid hipMalloc): x is in DEVICE memory (num_lat rows for
  * half = 0, num_lat-1 rows for half = 1, ld elements apart) and is filtered in
- * place.  The flagged rows of member 0's table are staged in a fixed 4 MiB
- * array of the library on the handle's device, so the call allocates nothing;
- * it returns GD_ERR_INVALID_ARG when flagged rows x pitch (num_lon rounded up
- * to 32) x 8 bytes exceed 4 MiB.  stream: a hipStream_t to enqueue on,
- * returning without waiting; NULL runs on the handle's stream and waits.
- * Every call on one device shares that array: calls that overlap on one
- * device (other streams, other threads, other handles) race. */
+ * place.  The flagged rows of member 0's table are filtered where they lie
+ * if x is 8-byte aligned and inside one allocation of the handle's device,
+ * and else staged in a fixed 4 MiB array of the library on that device, so the
+ * call allocates nothing; it returns GD_ERR_INVALID_ARG when flagged rows x
+ * pitch (num_lon rounded up to 32) x 8 bytes exceed 4 MiB, either way.
+ * stream: a hipStream_t to enqueue on, returning without waiting; NULL runs
+ * on the handle's stream and waits.  Every staged call on one device shares
+ * that array: staged calls that overlap on one device (other streams, other
+ * threads, other handles) race. */
 int gd_filter_rows_noalloc(gd_handle *h, int32_t half, double *x, int64_t ld, void *stream);
 
 /* Per-row filter table as set up by filter_init (filter_mod.F90:35-103):
