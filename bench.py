@@ -170,23 +170,27 @@ def _time_steps(d, steps, warmup):
     return time.perf_counter() - t0
 
 
-# the phase launch of each form that fused_phases() reports
-KERNEL_OF_FORM = {0: "k_tend", 1: "k_phase", 2: "k_wphase"}
+# the phase launch of each launch family of a step
+KERNEL_OF_FAMILY = {"tend": "k_tend", "phase": "k_phase", "wphase": "k_wphase", "rphase": "k_rphase"}
+
+
+def phase_kernel(prof):
+    """Kernel of the phase launches in a profile_kernels() result."""
+    return next(k for f, k in KERNEL_OF_FAMILY.items() if f in prof)
 
 
 def _kernel_us(d, reps):
-    """Replayed duration of the fast-pass second-predictor phase launch:
-    k_phase when the handle fuses phases, else k_tend."""
-    fused = d.fused_phases()
-    return d.time_kernel("phase" if fused else "tend", reps), fused
+    """Replayed duration of the step's fast-pass second-predictor phase launch
+    and its kernel (k_tend when the handle does not fuse phases)."""
+    us = d.time_kernel("phase" if d.fused_phases() else "tend", reps)
+    return us, phase_kernel(d.profile_kernels(1))
 
 
-def _tend_roofline(N, M, members, us, fused):
+def _tend_roofline(N, M, members, us, kname):
     """HBM roofline of the fast-pass second-predictor phase launch over all
     members (its algorithmic bytes over its replayed duration)."""
     nbytes = tend_launch_bytes(N, M, "mixed") * members
     achieved = nbytes / (us * 1e-6) / 1e9
-    kname = KERNEL_OF_FORM[fused]
     return {"bound": "hbm", "kernel": f"{kname}<float, fast pass> (second predictor)",
             "achieved": round(achieved, 1), "peak": 8000.0, "unit": "GB/s",
             "frac": round(achieved / 8000.0, 4),
@@ -596,7 +600,7 @@ def main():
     nbytes = tend_launch_bytes(N, M, "mixed")
     avg_s = mixed["kern_us"] * 1e-6
     achieved = nbytes / avg_s / 1e9
-    kname = KERNEL_OF_FORM[mixed["fused"]]
+    kname = phase_kernel(mixed["prof"])
     roofline = {"bound": "hbm",
                 "kernel": f"{kname}<float, fast pass> (second predictor" +
                           (": tendency + filter rows + epilogue)" if mixed["fused"] else ")"),

@@ -558,8 +558,10 @@ class Dycore:
 
     def fused_phases(self):
         """Form of the tendency phase launches: 0 a tendency launch then a
-        filter launch, 1 one fused launch (k_phase), 2 one fused launch with
-        a workgroup per row (k_wphase).  Nonzero means fused."""
+        filter launch, 1 one fused launch (k_phase), 2 one fused launch in
+        workgroups of two row tiles (k_wphase).  Nonzero means fused; calls
+        with strip tiles choose among the fused forms by their own size
+        (profile_kernels names the launches of a step)."""
         return int(lib().gd_fused_phases(self.h))
 
     def autotune(self, steps=40, cache=None):

@@ -373,6 +373,17 @@ int strip_form(const gd_handle *h) {
   return 1;
 }
 
+// The strip tiles of a call's phases for nm members, if it has any.
+bool set_strips(const gd_handle *h, Args &a, int pass, int nm) {
+  if (pass == GD_PASS_ALL || h->strip_b < h->strip_a || strip_rows(h) == 0) return false;
+  a.strip_a = h->strip_a;
+  a.strip_b = h->strip_b;
+  a.strip_r = strip_rows(h);
+  a.strip_ngroup = (h->strip_b - h->strip_a + a.strip_r) / a.strip_r;
+  a.nstrip = nm * a.strip_ngroup * a.nseg;
+  return true;
+}
+
 // One tendency phase (a.phase) of the active members with its filter rows:
 // one fused launch, or k_tend then k_filter.  strip: the rows strip_a..strip_b
 // run as strip tiles.
@@ -388,7 +399,7 @@ hipError_t enqueue_phase(gd_handle *h, Args a, int pass, bool in_full, bool stri
     return enqueue_filter(h, a);
   }
   set_fused(h, a, h->nact, strip ? h->near_far : h->far);
-  if (form == 3) return run(h, "phase", [&] { return launch_rphase(a, h->prec, pass, in_full, h->stream); });
+  if (form == 3) return run(h, "rphase", [&] { return launch_rphase(a, h->prec, pass, in_full, h->stream); });
   if (form == 2) return run(h, "wphase", [&] { return launch_wphase(a, h->prec, pass, in_full, h->stream); });
   return run(h, "phase", [&] { return launch_phase(a, h->prec, pass, in_full, h->stream); });
 }
@@ -432,14 +443,7 @@ hipError_t enqueue_call(gd_handle *h, double dt, int pass, int s0, int s_out, in
   a.hdt = dt * 0.5;
   hipError_t e;
   a.s0 = s0;
-  const bool strip = pass != GD_PASS_ALL && h->strip_b >= h->strip_a && strip_rows(h) > 0;
-  if (strip) {
-    a.strip_a = h->strip_a;
-    a.strip_b = h->strip_b;
-    a.strip_r = strip_rows(h);
-    a.strip_ngroup = (h->strip_b - h->strip_a + a.strip_r) / a.strip_r;
-    a.nstrip = h->nact * a.strip_ngroup * a.nseg;
-  }
+  const bool strip = set_strips(h, a, pass, h->nact);
   // first predictor: T = L(S0), S1 = S0 + dt/2 T
   a.phase = PH_A; a.s_in = s0; a.s_out = SP1;
   a.s_fold = before.slot;
@@ -1607,8 +1611,11 @@ int gd_time_kernel(gd_handle *h, int32_t kernel, int32_t reps, double *us) {
     }
     if (kernel == GD_TIME_PHASE) {
       Args f = a;
-      set_fused(h, f, h->nmem, h->far);
-      if (phase_form(h) == 2) return launch_wphase(f, h->prec, pass, false, h->stream);
+      const bool strip = set_strips(h, f, pass, h->nmem);
+      const int form = strip ? strip_form(h) : phase_form(h);
+      set_fused(h, f, h->nmem, strip ? h->near_far : h->far);
+      if (form == 3) return launch_rphase(f, h->prec, pass, false, h->stream);
+      if (form == 2) return launch_wphase(f, h->prec, pass, false, h->stream);
       return launch_phase(f, h->prec, pass, false, h->stream);
     }
     if (kernel == GD_TIME_FILTER_MM) {

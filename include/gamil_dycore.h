@@ -397,8 +397,8 @@ int64_t gd_device_bytes(const gd_handle *h);
  * state X is not modified).  kernel: GD_TIME_TEND (tendency kernel, fast
  * pass, second predictor), GD_TIME_FILTER (the filter of that phase),
  * GD_TIME_UPDATE (beta + corrector), GD_TIME_PHASE (that phase as one fused
- * launch, in the form gd_fused_phases reports: tendency, filter rows and
- * epilogue; GD_ERR_NOT_SUPPORTED when the handle steps with separate
+ * launch, in the form and with the strip tiles the step gives it: tendency,
+ * filter rows and epilogue; GD_ERR_NOT_SUPPORTED when the handle steps with separate
  * tendency and filter launches), GD_TIME_FILTER_MM
  * (the matrix-core projection of the momentum rows of every member; the
  * mixed_mfma and mixed_bf16 modes only).  No counterpart in the reference: a
@@ -417,11 +417,14 @@ enum { GD_TIME_TEND = 0, GD_TIME_FILTER = 1, GD_TIME_UPDATE = 2, GD_TIME_PHASE =
  * form.  In the calls of csp2 the rows away from the polar filter run as strip
  * tiles (several rows each) beside the launch's other rows, and the form is
  * then chosen by its filtered rows: 2, 1, or one fused launch with a workgroup
- * per filtered row (num_lon <= 1024), which this function reports as 1.
+ * per filtered row (num_lon <= 1024).  This function reports the form of the
+ * other launches (a forced or tuned 3 as 1); gd_profile_kernels names the
+ * launches of a step (phase, wphase, rphase).
  * GD_FUSED=0, 1, 2 or 3 in the environment when the handle is created forces
  * a form (2 falls back to 1 outside 255 to 762 longitudes; 3, the workgroup
  * per filtered row, to 1 where a launch cannot take it); GD_STRIP=n gives the
- * rows per strip tile (0: none).  Every form gives the same bits.  No
+ * rows per strip tile (0: none), GD_FOLD=0 or 1 whether such calls leave their
+ * update to the next call's first launch (by grid size when absent).  Every form gives the same bits.  No
  * counterpart in the reference. */
 int gd_fused_phases(const gd_handle *h);
 
