@@ -110,6 +110,7 @@ struct gd_handle {
   RowRanges near_all, near_far;
   void *dstrip = nullptr;
   int strip_mode = -1;   // rows per strip tile: -1 by launch size
+  int s2_mode = -1;      // strip tiles form S2 from Tb (use_s2_tb): -1 by batch size
   int fold_mode = -1;    // updates folded into the next call (use_fold): -1 by grid size
   int32_t *dstep = nullptr;
   double *ddiag = nullptr;  // [nmem][cap][3]
@@ -192,6 +193,7 @@ Args base_args(const gd_handle *h) {
   a.off_sy = h->off_sy;
   a.strip_coef = h->dstrip;
   a.s_fold = -1;
+  a.s2_hi = -1;
   a.nfar_rng = 1;
   a.nfar_rows = a.far_cnt[0] = h->M;
   a.mslots = h->dmslots;
@@ -421,7 +423,7 @@ struct Pending {
 // 1440x721 (4326) 0.730 / 0.747.  A launch of many rounds hides the k_update
 // gap and pays for the loads: 32 of 180x91 in k_phase (2912 tiles) 0.584 /
 // 0.568, but 8 of 720x361 (8664) 1.485 / 1.546 and 64 of 360x181 (23168) 3.757 /
-// 3.850.  k_rphase, with no registers left for it, keeps k_update.
+// 3.850.  k_rphase, which serves such launches, keeps k_update.
 bool use_fold(const gd_handle *h) {
   if (h->strip_b < h->strip_a || strip_rows(h) == 0) return false;
   const int form = strip_form(h);
@@ -429,6 +431,24 @@ bool use_fold(const gd_handle *h) {
   if (h->fold_mode >= 0) return h->fold_mode != 0;
   const int64_t entries = (int64_t)h->M * ((h->N + kSeg - 1) / kSeg);
   return entries <= 6 * kBlock && h->nact * entries <= 16 * (int64_t)h->ncu;
+}
+
+// Whether the strip tiles of a call's phase C form S2 = S0 + hdt Tb where they
+// read it, so that phase B stores S2 only next to other tiles (GD_S2TB = 0 or
+// 1 in the environment when the handle is created overrides): three field
+// stores fewer per call, for loads of two fields in place of one in phase C.
+// It pays where a call's fields (three each of S0, S1, S2, Tb, Tc, and ghs) no
+// longer stay in the 256 MB memory-side cache.  ms per step without and with:
+// 24 of 360x181 (214 MB) 1.168 / 1.088, 64 of them (570 MB) 3.328 / 3.277, 6 of
+// 720x361 (204 MB) 1.036 / 1.004, 8 of them (272 MB) 1.417 / 1.349, 128 of
+// 180x91 (286 MB) 1.727 / 1.633, 2 of 1440x721 (266 MB) 1.510 / 1.433; below,
+// the loads cost more than the stores: 16 of 360x181 (142 MB) 0.758 / 0.768, 4 of
+// 720x361 (136 MB) 0.706 / 0.721, one 1440x721 (133 MB) 0.730 / 0.760.
+bool use_s2_tb(const gd_handle *h) {
+  const int form = strip_form(h);
+  if (form != 1 && form != 3) return false;
+  if (h->s2_mode >= 0) return h->s2_mode != 0;
+  return (int64_t)16 * h->nact * h->M * h->P * (int64_t)sizeof(double) > ((int64_t)160 << 20);
 }
 
 // predict_correct(dt, s0 -> s_out, pass) (dycore_mod.F90:754-792).  before: s0
@@ -452,6 +472,11 @@ hipError_t enqueue_call(gd_handle *h, double dt, int pass, int s0, int s_out, in
   if ((e = enqueue_phase(h, a, pass, s0 == SX, strip)) != hipSuccess) return e;
   a.s_fold = -1;
   // second predictor: T = L(S1), S2 = S0 + dt/2 T, keep T
+  if (strip && use_s2_tb(h)) {
+    a.s2_tb = 1;
+    a.s2_lo = a.strip_a + 2;
+    a.s2_hi = a.strip_b - 2;
+  }
   a.phase = PH_B; a.s_in = SP1; a.s_out = SP2;
   if ((e = enqueue_phase(h, a, pass, false, strip)) != hipSuccess) return e;
   // corrector tendency T = L(S2) and the beta inner-product partials
@@ -1010,6 +1035,8 @@ int gd_create(const gd_config *cfg, int32_t n_members, gd_handle **out) {
     h->fused_mode = env && env[0] >= '0' && env[0] <= '3' ? env[0] - '0' : -1;
     const char *bd = std::getenv("GD_STRIP");
     if (bd && bd[0]) h->strip_mode = std::max(0, std::min(std::atoi(bd), 32));
+    const char *s2 = std::getenv("GD_S2TB");
+    if (s2 && s2[0] >= '0' && s2[0] <= '1' && s2[1] == 0) h->s2_mode = s2[0] - '0';
     const char *fo = std::getenv("GD_FOLD");
     if (fo && fo[0] >= '0' && fo[0] <= '1' && fo[1] == 0) h->fold_mode = fo[0] - '0';
     const char *nar = std::getenv("GD_UPD_NARROW");

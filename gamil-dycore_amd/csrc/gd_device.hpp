@@ -154,6 +154,9 @@ struct Args {
   // beta from the partials with fold_qcon, its step fold_dt
   int s_fold, fold_qcon;
   double fold_dt;
+  // a call whose strip tiles form S2 = S0 + hdt Tb in phase C (s2_tb): its
+  // phase B strips do not store S2 in rows s2_lo..s2_hi
+  int s2_tb, s2_lo, s2_hi;
   const void *strip_coef;
   int in_full;                 // k_diffuse: read stored u, v of s_in
   int nslots;

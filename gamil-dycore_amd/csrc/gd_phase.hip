@@ -132,7 +132,8 @@ __device__ __forceinline__ void near_tile(const Args &a, const FiltRow fr, unsig
 template <int KP, bool STRIP>
 constexpr int phase_waves() { return KP == 4 ? (STRIP ? 4 : 5) : 3; }
 
-template <typename CT, int PASS, bool IN_FULL, int KP, bool STRIP, bool FOLD = false>
+// S2TB: the strip tiles of a phase C that form S2 from Tb (strip_tile).
+template <typename CT, int PASS, bool IN_FULL, int KP, bool STRIP, bool FOLD = false, bool S2TB = false>
 __global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(phase_waves<KP, STRIP>(), 8)))
 k_phase(const Args a) {
   extern __shared__ __align__(16) unsigned char smem[];
@@ -150,7 +151,7 @@ k_phase(const Args a) {
   }
   if constexpr (STRIP) {
     if (b >= a.nnear_pad + a.row_blk) {
-      strip_block<CT, PASS, IN_FULL, 1, FOLD>(a, a.nnear_pad + a.row_blk, smem, red);
+      strip_block<CT, PASS, IN_FULL, 1, S2TB ? 2 : (FOLD ? 1 : 0)>(a, a.nnear_pad + a.row_blk, smem, red);
       return;
     }
   }
@@ -366,7 +367,7 @@ __device__ __forceinline__ void rnear_block(const Args &a, int t, unsigned char 
   filter_wave<CT, KQ>(a, mb, fr, tw, b0 + fr.comp * L, b1 + fr.comp * L, PASS == 2 && fr.comp == CDGD);
 }
 
-template <typename CT, int PASS, bool IN_FULL, int KQ>
+template <typename CT, int PASS, bool IN_FULL, int KQ, bool S2TB = false>
 __global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(KQ == 8 ? 4 : 3, 8)))
 k_rphase(const Args a) {
   extern __shared__ __align__(16) unsigned char smem[];
@@ -378,7 +379,7 @@ k_rphase(const Args a) {
     return;
   }
   if (b >= a.nnear_pad + a.row_blk) {
-    strip_block<CT, PASS, IN_FULL>(a, a.nnear_pad + a.row_blk, smem, red);
+    strip_block<CT, PASS, IN_FULL, 1, S2TB ? 2 : 0>(a, a.nnear_pad + a.row_blk, smem, red);
     return;
   }
   const int bb = b - a.nnear_pad, t = (bb % kXcd) * (a.row_blk / kXcd) + bb / kXcd;
@@ -492,6 +493,12 @@ static hipError_t launch_phase_k(Args a, int pass, bool in_full, hipStream_t s) 
       hipLaunchKernelGGL((k_phase<CT, 1, false, KP, true, true>), g, b, lds, s, a);
     else
       hipLaunchKernelGGL((k_phase<CT, 2, false, KP, true, true>), g, b, lds, s, a);
+  } else if (a.s2_tb && a.phase == PH_C) {
+    if (pass == 0 || in_full || a.nstrip <= 0) return hipErrorInvalidValue;
+    if (pass == 1)
+      hipLaunchKernelGGL((k_phase<CT, 1, false, KP, true, false, true>), g, b, lds, s, a);
+    else
+      hipLaunchKernelGGL((k_phase<CT, 2, false, KP, true, false, true>), g, b, lds, s, a);
   } else if (a.nstrip > 0) {
     if (pass == 0) return hipErrorInvalidValue;
     if (pass == 1) { if (in_full) GD_PH(1, true, true); else GD_PH(1, false, true); }
@@ -520,7 +527,14 @@ static hipError_t launch_rphase_k(Args a, int pass, bool in_full, hipStream_t s)
   dim3 g(a.nnear_pad + a.row_blk + a.strip_blk), b(kBlock);
   const size_t lds = rphase_lds<CT>(a.N, a.fft_L);
 #define GD_PH(P, F) hipLaunchKernelGGL((k_rphase<CT, P, F, KQ>), g, b, lds, s, a)
-  if (pass == 1) { if (in_full) GD_PH(1, true); else GD_PH(1, false); }
+  if (a.s2_tb && a.phase == PH_C) {
+    if (in_full || a.nstrip <= 0) return hipErrorInvalidValue;
+    if (pass == 1)
+      hipLaunchKernelGGL((k_rphase<CT, 1, false, KQ, true>), g, b, lds, s, a);
+    else
+      hipLaunchKernelGGL((k_rphase<CT, 2, false, KQ, true>), g, b, lds, s, a);
+  }
+  else if (pass == 1) { if (in_full) GD_PH(1, true); else GD_PH(1, false); }
   else { if (in_full) GD_PH(2, true); else GD_PH(2, false); }
 #undef GD_PH
   return hipGetLastError();
@@ -542,7 +556,8 @@ size_t rphase_lds_bytes(int N, int L, int prec) {
 template <typename CT, int KQ>
 static hipError_t configure_rphase_k(int max_lds) {
   const void *fns[] = {(const void *)k_rphase<CT, 1, true, KQ>, (const void *)k_rphase<CT, 1, false, KQ>,
-                       (const void *)k_rphase<CT, 2, true, KQ>, (const void *)k_rphase<CT, 2, false, KQ>};
+                       (const void *)k_rphase<CT, 2, true, KQ>, (const void *)k_rphase<CT, 2, false, KQ>,
+                       (const void *)k_rphase<CT, 1, false, KQ, true>, (const void *)k_rphase<CT, 2, false, KQ, true>};
   for (const void *f : fns) {
     hipError_t e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, max_lds);
     if (e != hipSuccess) return e;
@@ -609,7 +624,9 @@ static hipError_t configure_phase_k(int max_lds) {
                        (const void *)k_phase<CT, 2, true, KP, false>, (const void *)k_phase<CT, 2, false, KP, false>,
                        (const void *)k_phase<CT, 1, true, KP, true>,  (const void *)k_phase<CT, 1, false, KP, true>,
                        (const void *)k_phase<CT, 2, true, KP, true>,  (const void *)k_phase<CT, 2, false, KP, true>,
-                       (const void *)k_phase<CT, 1, false, KP, true, true>, (const void *)k_phase<CT, 2, false, KP, true, true>};
+                       (const void *)k_phase<CT, 1, false, KP, true, true>, (const void *)k_phase<CT, 2, false, KP, true, true>,
+                       (const void *)k_phase<CT, 1, false, KP, true, false, true>,
+                       (const void *)k_phase<CT, 2, false, KP, true, false, true>};
   for (const void *f : fns) {
     hipError_t e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, max_lds);
     if (e != hipSuccess) return e;

@@ -120,9 +120,10 @@ __host__ __device__ constexpr size_t strip_lds_bytes(int rows) { return (size_t)
 
 // Phase a.phase (PH_A, PH_B or PH_C) of tile t = (member, group of a.strip_r
 // rows, segment), segment fastest.  live = false: no stores (a spare tile).
-// FOLD: phase A's state is s_fold + dt beta Tc, formed where a row is loaded,
-// and stored to s_in.  `red`: 24 doubles.
-template <typename CT, int PASS, bool FULL, bool FOLD>
+// FOLD 1: phase A's state is s_fold + dt beta Tc, formed where a row is loaded,
+// and stored to s_in.  FOLD 2: phase C's state is S0 + hdt Tb, which phase B
+// then need not have stored.  `red`: 24 doubles.
+template <typename CT, int PASS, bool FULL, int FOLD>
 __device__ __forceinline__ void strip_tile(const Args &a, int t, bool live, unsigned char *smem, double *red) {
   const int N = a.N, nseg = a.nseg, tid = ltid(), lane = threadIdx.x & 63, wv = (threadIdx.x >> 6) & 3;
   const int seg = t % nseg, q = t / nseg, grp = q % a.strip_ngroup, m = q / a.strip_ngroup;
@@ -131,7 +132,7 @@ __device__ __forceinline__ void strip_tile(const Args &a, int t, bool live, unsi
   const int i0 = seg * kSeg, W = min(N - i0, kSeg);
   const bool first = lane == 0, last = lane == 63, pc = a.phase == PH_C;
   double *sums = (double *)smem;
-  const double dtb = FOLD ? fold_step(a, mb, red) : 0.0;
+  const double dtb = FOLD == 1 ? fold_step(a, mb, red) : (FOLD == 2 ? a.hdt : 0.0);
   // (a wave past the segment's end has nothing to do but its zero sums)
   const bool busy = __builtin_amdgcn_readfirstlane(wv * 64) < W;
   if (busy) {
@@ -144,9 +145,10 @@ __device__ __forceinline__ void strip_tile(const Args &a, int t, bool live, unsi
     // is inside the row)
     const int ic = i0 + min(tid, W + 1);
     const unsigned c0 = wrap(ic), cx = wrap(ic + (last ? 1 : (first ? -1 : 0)));
-    const int si = FOLD ? a.s_fold : a.s_in;
+    const int si = FOLD == 1 ? a.s_fold : (FOLD == 2 ? a.s0 : a.s_in);
     const double *gd = mb.st(si, FGD), *Ug = mb.st(si, FU), *Vg = mb.st(si, FV), *hg = mb.ghs();
-    const double *tg = mb.tc(CDGD), *tu = mb.tc(CDU), *tv = mb.tc(CDV);
+    const double *tg = FOLD == 2 ? mb.tb(CDGD) : mb.tc(CDGD), *tu = FOLD == 2 ? mb.tb(CDU) : mb.tc(CDU);
+    const double *tv = FOLD == 2 ? mb.tb(CDV) : mb.tc(CDV);
     auto in = [&](const double *f, const double *tc, unsigned o) {
       if constexpr (FOLD) return ld(f, o) + dtb * ld(tc, o);
       return ld(f, o);
@@ -173,14 +175,16 @@ __device__ __forceinline__ void strip_tile(const Args &a, int t, bool live, unsi
           pq[4] += xg * dg * c.fcos;
           pq[5] += dg * dg * c.fcos;
         } else {
-          if (FOLD) {
+          if (FOLD == 1) {
             st(mb.st(a.s_in, FU), o, xu);
             st(mb.st(a.s_in, FV), o, xv);
             st(mb.st(a.s_in, FGD), o, xg);
           }
-          st(ou, o, xu + a.hdt * du);
-          st(ov, o, xv + a.hdt * dv);
-          st(og, o, xg + a.hdt * dg);
+          if (a.phase != PH_B || j < a.s2_lo || j > a.s2_hi) {
+            st(ou, o, xu + a.hdt * du);
+            st(ov, o, xv + a.hdt * dv);
+            st(og, o, xg + a.hdt * dg);
+          }
           if (a.phase == PH_B) {
             st(mb.tb(CDU), o, du);
             st(mb.tb(CDV), o, dv);
@@ -248,7 +252,8 @@ __device__ __forceinline__ void strip_tile(const Args &a, int t, bool live, unsi
       }
       for (int j = r0; j <= r1; ++j) {
         const unsigned o = (unsigned)j * P8 + c0;
-        const double xu = FOLD ? s.U : ld(pu, o), xv = FOLD ? s.V : ld(pv, o), xg = FOLD ? s.gd : ld(pg, o);
+        const double xu = FOLD == 1 ? s.U : ld(pu, o), xv = FOLD == 1 ? s.V : ld(pv, o);
+        const double xg = FOLD == 1 ? s.gd : ld(pg, o);
         const Ld l = l2;
         l2 = load(min(j + 2, r1 + 1));
         const StripRow<CT> cn = strip_row<CT>(a, j + 1);
@@ -344,8 +349,8 @@ __device__ __forceinline__ void strip_tile(const Args &a, int t, bool live, unsi
       CT Up = p.U, Vp = p.V, Yp = p.Y, Zp = p.Z;
       for (int j = r0; j <= r1; ++j) {
         const unsigned o = (unsigned)j * P8 + c0;
-        const double xu = FOLD ? in(Ug, tu, o) : ld(pu, o), xv = FOLD ? in(Vg, tv, o) : ld(pv, o);
-        const double xg = FOLD ? in(gd, tg, o) : ld(pg, o);
+        const double xu = FOLD == 1 ? in(Ug, tu, o) : ld(pu, o), xv = FOLD == 1 ? in(Vg, tv, o) : ld(pv, o);
+        const double xg = FOLD == 1 ? in(gd, tg, o) : ld(pg, o);
         const Ld l = l0;
         l0 = load(min(j + 2, r1 + 1));
         const StripRow<CT> cn = strip_row<CT>(a, j + 1);
@@ -382,7 +387,7 @@ __device__ __forceinline__ void strip_tile(const Args &a, int t, bool live, unsi
 // in each, every XCD a contiguous run (base and strip_blk are multiples of
 // kXcd).  A spare tile past the last does the last one's work and barriers
 // without its stores.
-template <typename CT, int PASS, bool FULL, int TILES = 1, bool FOLD = false>
+template <typename CT, int PASS, bool FULL, int TILES = 1, int FOLD = 0>
 __device__ __forceinline__ void strip_block(const Args &a, int base, unsigned char *smem, double *red) {
   const int b = (int)blockIdx.x - base;
   const int t0 = ((b % kXcd) * (a.strip_blk / kXcd) + b / kXcd) * TILES;

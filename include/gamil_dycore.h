@@ -424,7 +424,9 @@ enum { GD_TIME_TEND = 0, GD_TIME_FILTER = 1, GD_TIME_UPDATE = 2, GD_TIME_PHASE =
  * a form (2 falls back to 1 outside 255 to 762 longitudes; 3, the workgroup
  * per filtered row, to 1 where a launch cannot take it); GD_STRIP=n gives the
  * rows per strip tile (0: none), GD_FOLD=0 or 1 whether such calls leave their
- * update to the next call's first launch (by grid size when absent).  Every form gives the same bits.  No
+ * update to the next call's first launch (by grid size when absent), GD_S2TB=0 or
+ * 1 whether their strip tiles form the second predictor again in the corrector
+ * phase instead of loading it (by batch size when absent).  Every form gives the same bits.  No
  * counterpart in the reference. */
 int gd_fused_phases(const gd_handle *h);
 
