@@ -1400,6 +1400,10 @@ int gd_filter_rows_noalloc(gd_handle *h, int32_t half, double *x, int64_t ld, vo
                     std::to_string(h->P) + " doubles need " + std::to_string(need) + " bytes of scratch, more than " +
                     std::to_string(kScratchBytes));
   if (rows.empty()) return GD_OK;
+  // (byte offsets of the rows have to fit 64 bits: past that they would wrap
+  // into memory that is not the caller's)
+  if (ld > (INT64_MAX / (int64_t)sizeof(double) - h->N) / h->M)
+    return fail(h, GD_ERR_INVALID_ARG, "gd_filter_rows_noalloc: ld too large");
   hipSetDevice(h->device);
   hipStream_t s = stream ? (hipStream_t)stream : h->stream;
   const size_t P = h->P, N = h->N;

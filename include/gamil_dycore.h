@@ -177,7 +177,8 @@ int gd_filter_rows(gd_handle *h, int32_t half, double *x, int64_t ld);
  * if x is 8-byte aligned and inside one allocation of the handle's device,
  * and else staged in a fixed 4 MiB array of the library on that device, so the
  * call allocates nothing; it returns GD_ERR_INVALID_ARG when flagged rows x
- * pitch (num_lon rounded up to 32) x 8 bytes exceed 4 MiB, either way.
+ * pitch (num_lon rounded up to 32) x 8 bytes exceed 4 MiB, either way, or
+ * when num_lat x ld x 8 bytes do not fit 63 bits.
  * stream: a hipStream_t to enqueue on, returning without waiting; NULL runs
  * on the handle's stream and waits.  Every staged call on one device shares
  * that array: staged calls that overlap on one device (other streams, other
