@@ -1529,6 +1529,7 @@ int gd_autotune(gd_handle *h, int32_t steps, const char *cache_path, int32_t *fu
                  (bf == 3 && !h->rphase_ok)))
     cached = false;
   if (!cached) {
+    bf = bw = -1;  // (nothing of a refused entry is kept)
     // fused or separate phase launches (both give the same bits; a forced
     // GD_FUSED keeps its form) ...
     std::vector<int> fopts;
