@@ -567,8 +567,9 @@ class Dycore:
     def autotune(self, steps=40, cache=None):
         """Pick the fastest launch shapes for the current active-member count
         (gd_autotune; results stay bit for bit those of the defaults).
-        Returns {'fused', 'form', 'upd_wpm', 'ms_per_step', 'cache'}: 'form' as
-        fused_phases() reports it, 'fused' whether that form is fused."""
+        Returns {'fused', 'form', 'upd_wpm', 'ms_per_step', 'cache'}: 'form' the
+        form a step now has (0 separate launches, 1 k_phase, 2 k_wphase, 3
+        k_rphase), 'fused' whether that form is fused."""
         f, w, ms = C.c_int32(0), C.c_int32(0), C.c_double(0.0)
         _check(lib().gd_autotune(self.h, int(steps), None if cache is None else str(cache).encode(),
                                  C.byref(f), C.byref(w), C.byref(ms)), self.h)

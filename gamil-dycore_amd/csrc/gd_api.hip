@@ -125,8 +125,8 @@ struct gd_handle {
   double *scratch = nullptr;
   std::string scratch_err;
   // autotuned launch shapes per active-member count (gd_autotune): phase
-  // launch form (0 separate, 1 k_phase, 2 k_wphase), k_update workgroups
-  // per member
+  // launch form (0 separate, 1 k_phase, 2 k_wphase, 3 k_rphase), k_update
+  // workgroups per member
   std::map<int, int> tuned_fused, tuned_wpm;
   std::vector<int> prow[2];
   FiltRow *dprow[2] = {nullptr, nullptr};
@@ -348,6 +348,9 @@ int strip_rows(const gd_handle *h) {
   return h->nact * nseg * ((far + 1) / 2) <= 2 * (int64_t)h->ncu ? 2 : 4;
 }
 
+// Whether the fast and slow calls have strip tiles.
+bool has_strips(const gd_handle *h) { return h->strip_b >= h->strip_a && strip_rows(h) != 0; }
+
 // Form of the phase launches of a call with strip tiles, unless the handle's
 // form is forced or tuned: 1 k_phase, 2 k_wphase, 3 k_rphase.
 // k_wphase (shortest chain of a filter row) while its workgroups fit about two
@@ -375,9 +378,14 @@ int strip_form(const gd_handle *h) {
   return 1;
 }
 
+// Form of the phase launches of a step's calls.
+int step_form(const gd_handle *h) {
+  return h->cfg.split_scheme == GD_SPLIT_CSP2 && has_strips(h) ? strip_form(h) : phase_form(h);
+}
+
 // The strip tiles of a call's phases for nm members, if it has any.
 bool set_strips(const gd_handle *h, Args &a, int pass, int nm) {
-  if (pass == GD_PASS_ALL || h->strip_b < h->strip_a || strip_rows(h) == 0) return false;
+  if (pass == GD_PASS_ALL || !has_strips(h)) return false;
   a.strip_a = h->strip_a;
   a.strip_b = h->strip_b;
   a.strip_r = strip_rows(h);
@@ -425,7 +433,7 @@ struct Pending {
 // 0.568, but 8 of 720x361 (8664) 1.485 / 1.546 and 64 of 360x181 (23168) 3.757 /
 // 3.850.  k_rphase, which serves such launches, keeps k_update.
 bool use_fold(const gd_handle *h) {
-  if (h->strip_b < h->strip_a || strip_rows(h) == 0) return false;
+  if (!has_strips(h)) return false;
   const int form = strip_form(h);
   if (form != 1 && form != 2) return false;
   if (h->fold_mode >= 0) return h->fold_mode != 0;
@@ -887,14 +895,21 @@ void drop_graphs(gd_handle *h) {
   h->graph_failed = false;
 }
 
-// Autotuner cache key: everything that decides the launch shapes' timing.
+// Autotuner cache key: everything that decides the launch shapes' timing, the
+// settings forced in the environment among it.  v goes up whenever the rules
+// or kernels behind a form change, so that an entry of an earlier library is
+// timed again.
+constexpr int kTuneVersion = 2;
+
 std::string tune_key(const gd_handle *h, const char *arch) {
   const gd_config &c = h->cfg;
-  char b[320];
+  char b[400];
   std::snprintf(b, sizeof b,
-                "arch=%s N=%d M=%d members=%d active=%d prec=%d split=%d sub=%d adv=%d diff=%d filt=%zu",
+                "arch=%s N=%d M=%d members=%d active=%d prec=%d split=%d sub=%d adv=%d diff=%d filt=%zu"
+                " v=%d form=%d strip=%d fold=%d s2tb=%d narrow=%d",
                 arch, h->N, h->M, h->nmem, h->nact, h->prec, c.split_scheme, c.subcycles, c.uv_adv_scheme,
-                c.use_diffusion ? c.diffusion_order : 0, h->frows.size() / (size_t)h->nmem);
+                c.use_diffusion ? c.diffusion_order : 0, h->frows.size() / (size_t)h->nmem, kTuneVersion,
+                h->fused_mode, h->strip_mode, h->fold_mode, h->s2_mode, h->upd_narrow);
   return b;
 }
 
@@ -1524,23 +1539,24 @@ int gd_autotune(gd_handle *h, int32_t steps, const char *cache_path, int32_t *fu
   int bf = -1, bw = -1;
   double bms = 0.0;
   if (cache_path && !cache_path[0]) cache_path = nullptr;  // "" : no cache
+  // a workgroup per filtered row needs calls with strip tiles
+  const bool rows_ok = h->rphase_ok && h->cfg.split_scheme == GD_SPLIT_CSP2 && has_strips(h);
   bool cached = cache_path && tune_lookup(cache_path, key, bf, bw, bms);
   if (cached && (bw < 1 || bw > h->M || bf < 0 || bf > 3 || (bf && !h->fused_ok) || (bf == 2 && !h->wide_ok) ||
-                 (bf == 3 && !h->rphase_ok)))
+                 (bf == 3 && !rows_ok)))
     cached = false;
   if (!cached) {
     bf = bw = -1;  // (nothing of a refused entry is kept)
     // fused or separate phase launches (both give the same bits; a forced
-    // GD_FUSED keeps its form) ...
+    // GD_FUSED keeps the form a step has under it) ...
     std::vector<int> fopts;
     if (h->fused_mode >= 0 || !h->fused_ok)
-      fopts = {phase_form(h)};
+      fopts = {step_form(h)};
     else if (h->wide_ok)
       fopts = {0, 1, 2};
     else
       fopts = {0, 1};
-    if (h->fused_mode < 0 && h->rphase_ok && h->strip_b >= h->strip_a && h->cfg.split_scheme == GD_SPLIT_CSP2)
-      fopts.push_back(3);
+    if (h->fused_mode < 0 && rows_ok) fopts.push_back(3);
     // ... and k_update rows per workgroup (each workgroup forms its member's
     // beta from all of the member's partials in one order: the same bits)
     std::vector<int> wopts;

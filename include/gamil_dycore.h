@@ -433,16 +433,18 @@ int gd_fused_phases(const gd_handle *h);
 
 /* Tile autotuner (no counterpart in the reference).  For the current
  * active-member count, times `steps` steps (1..512) of every launch shape
- * that cannot change a result -- the form of the phase launches (separate
- * tendency and filter launches, fused, fused with a workgroup per row; see
- * gd_fused_phases), and the workgroups per member of the corrector update --
- * from the members' current state, puts that state back, and keeps the
- * fastest shape for later gd_step calls at this active-member count (the
- * results are bit for bit those of the default shapes).  cache_path (may be
- * NULL) is a text file of earlier results keyed by the device architecture,
- * grid, member counts, precision and schemes: a cached entry is applied
- * without timing, a new result is appended.  Outputs (may be NULL): the
- * chosen form (0 to 3, as GD_FUSED names them), workgroups per member and milliseconds per
+ * that cannot change a result -- the form of the phase launches (0 to 3, see
+ * gd_fused_phases; 3 only for csp2 steps with strip tiles), and the workgroups
+ * per member of the corrector update -- from the members' current state, puts
+ * that state back, and keeps the fastest shape for later gd_step calls at this
+ * active-member count (the results are bit for bit those of the default
+ * shapes).  A form forced by GD_FUSED is the only candidate.  cache_path (may
+ * be NULL) is a text file of earlier results keyed by the device architecture,
+ * grid, member counts, precision, schemes, the settings forced in the
+ * environment and a version of the launch rules: a cached entry is applied
+ * without timing, a new result is appended, and entries of a library with
+ * other rules are not used.  Outputs (may be NULL): the form a step now has (0
+ * to 3, as GD_FUSED names them), workgroups per member and milliseconds per
  * step. */
 int gd_autotune(gd_handle *h, int32_t steps, const char *cache_path, int32_t *fused,
                 int32_t *upd_wpm, double *ms_per_step);
