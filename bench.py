@@ -38,16 +38,31 @@ ENS = dict(N=360, M=181, dt=240.0, coef=1.0e5, members=64,
                    pert_rms=5.0))
 
 
-def tend_launch_bytes(N, M, prec):
+def tend_launch_bytes(N, M, prec, unstored=0):
     """Algorithmic HBM bytes of one launch of the tendency kernel in the
     second predictor of a fast-pass call (S2 = S0 + dt/2 L(S1), keep Tb):
-    read S1 (gd, U, V), ghs and S0 (gd, U, V); write S2 (gd, U, V) and Tb
-    (du, dv, dgd).  gd, U, u live on N x M full rows, V on N x (M-1) half
-    rows; state and stored tendencies are FP64 in both precision modes."""
+    read S1 (gd, U, V), ghs and S0 (gd, U, V); write S2 (gd, U, V; not in
+    `unstored` rows) and Tb (du, dv, dgd).  gd, U, u live on N x M full rows,
+    V on N x (M-1) half rows; state and stored tendencies are FP64 in both
+    precision modes."""
     full, half = N * M, N * (M - 1)
     state = 8 * (full + full + half)            # gd, U, V
     tend = 8 * (full + half) + 8 * full         # du, dv, dgd
-    return state + 8 * full + state + state + tend
+    return state + 8 * full + state + state + tend - 3 * 8 * N * unstored
+
+
+def unstored_rows(d, prof):
+    """Rows of S2 that the second predictor's launch does not store: none, or
+    where the corrector's strip tiles form it again (a *_s2tb launch) the rows
+    of the strip tiles but the two next to other tiles at each end."""
+    if not any(f.endswith("_s2tb") for f in prof):
+        return 0
+    full, half, _, _ = d.filter_table()
+    best = run = 0
+    for j in range(2, d.M - 3):
+        run = 0 if full[j] or half[j] else run + 1
+        best = max(best, run)
+    return max(0, best - 4)
 
 
 def traffic_from_profile(kernel, grid="720x361"):
@@ -94,8 +109,8 @@ def run_gpu(gd, prec, ic, steps, warmup, repeats):
         d.step(int(full))
         lat.append(time.perf_counter() - s0)
     prof = d.profile_kernels(60)
-    fused = d.fused_phases()
-    kern_us = d.time_kernel("phase" if fused else "tend", 200)
+    kern_us, kname, _ = _kernel_us(d, 200)
+    fused = kname != "k_tend"
     d.close()
     return dict(elapsed=elapsed, mass=mass[:, 0], energy=energy[:, 0], lat=lat, prof=prof, cut=cut,
                 kern_us=kern_us, fused=fused)
@@ -180,16 +195,18 @@ def phase_kernel(prof):
 
 
 def _kernel_us(d, reps):
-    """Replayed duration of the step's fast-pass second-predictor phase launch
-    and its kernel (k_tend when the handle does not fuse phases)."""
-    us = d.time_kernel("phase" if d.fused_phases() else "tend", reps)
-    return us, phase_kernel(d.profile_kernels(1))
+    """Replayed duration of the step's fast-pass second-predictor phase launch,
+    its kernel (k_tend when the step does not fuse phases) and the rows of S2
+    it does not store."""
+    prof = d.profile_kernels(1)
+    kname = phase_kernel(prof)
+    return d.time_kernel("tend" if kname == "k_tend" else "phase", reps), kname, unstored_rows(d, prof)
 
 
-def _tend_roofline(N, M, members, us, kname):
+def _tend_roofline(N, M, members, us, kname, unstored):
     """HBM roofline of the fast-pass second-predictor phase launch over all
     members (its algorithmic bytes over its replayed duration)."""
-    nbytes = tend_launch_bytes(N, M, "mixed") * members
+    nbytes = tend_launch_bytes(N, M, "mixed", unstored) * members
     achieved = nbytes / (us * 1e-6) / 1e9
     return {"bound": "hbm", "kernel": f"{kname}<float, fast pass> (second predictor)",
             "achieved": round(achieved, 1), "peak": 8000.0, "unit": "GB/s",

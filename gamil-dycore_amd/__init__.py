@@ -557,11 +557,11 @@ class Dycore:
         write_restart(path, u, v, gd, self._ghs[member], **info)
 
     def fused_phases(self):
-        """Form of the tendency phase launches: 0 a tendency launch then a
-        filter launch, 1 one fused launch (k_phase), 2 one fused launch in
-        workgroups of two row tiles (k_wphase).  Nonzero means fused; calls
-        with strip tiles choose among the fused forms by their own size
-        (profile_kernels names the launches of a step)."""
+        """Form of the tendency phase launches without strip tiles: 0 a
+        tendency launch then a filter launch, 1 one fused launch (k_phase), 2
+        one fused launch in workgroups of two row tiles (k_wphase).  Nonzero
+        means fused.  The calls of csp2 with strip tiles choose their form by
+        their own size: profile_kernels names the launches of a step."""
         return int(lib().gd_fused_phases(self.h))
 
     def autotune(self, steps=40, cache=None):
@@ -582,7 +582,7 @@ class Dycore:
     def time_kernel(self, kernel, reps=200):
         """Microseconds per launch of one kernel replayed back to back:
         kernel 'tend' (fast pass, second predictor), 'filter', 'update',
-        'phase' (that phase as one fused launch; fused handles only) or
+        'phase' (that phase as one fused launch; steps with fused phases only) or
         'filter_mm' (the matrix-core projection of the momentum rows; the
         mixed_mfma and mixed_bf16 modes only)."""
         us = C.c_double(0.0)

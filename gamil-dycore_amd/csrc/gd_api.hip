@@ -409,9 +409,12 @@ hipError_t enqueue_phase(gd_handle *h, Args a, int pass, bool in_full, bool stri
     return enqueue_filter(h, a);
   }
   set_fused(h, a, h->nact, strip ? h->near_far : h->far);
-  if (form == 3) return run(h, "rphase", [&] { return launch_rphase(a, h->prec, pass, in_full, h->stream); });
+  const bool tb = a.s2_tb && a.phase == PH_C;
+  if (form == 3)
+    return run(h, tb ? "rphase_s2tb" : "rphase",
+               [&] { return launch_rphase(a, h->prec, pass, in_full, h->stream); });
   if (form == 2) return run(h, "wphase", [&] { return launch_wphase(a, h->prec, pass, in_full, h->stream); });
-  return run(h, "phase", [&] { return launch_phase(a, h->prec, pass, in_full, h->stream); });
+  return run(h, tb ? "phase_s2tb" : "phase", [&] { return launch_phase(a, h->prec, pass, in_full, h->stream); });
 }
 
 // The call before, whose state s0 + dt beta Tc -> s_out a call's phase A forms
@@ -459,6 +462,16 @@ bool use_s2_tb(const gd_handle *h) {
   return (int64_t)16 * h->nact * h->M * h->P * (int64_t)sizeof(double) > ((int64_t)160 << 20);
 }
 
+// Phases B and C of a call with strip tiles: S2 formed again in phase C where
+// use_s2_tb says so, and stored by phase B only in the rows that other tiles read
+// too.
+void set_s2(const gd_handle *h, Args &a) {
+  if (!use_s2_tb(h)) return;
+  a.s2_tb = 1;
+  a.s2_lo = a.strip_a + 2;
+  a.s2_hi = a.strip_b - 2;
+}
+
 // predict_correct(dt, s0 -> s_out, pass) (dycore_mod.F90:754-792).  before: s0
 // is still to be formed from this call; leave: the update is left to the next
 // call.
@@ -480,11 +493,7 @@ hipError_t enqueue_call(gd_handle *h, double dt, int pass, int s0, int s_out, in
   if ((e = enqueue_phase(h, a, pass, s0 == SX, strip)) != hipSuccess) return e;
   a.s_fold = -1;
   // second predictor: T = L(S1), S2 = S0 + dt/2 T, keep T
-  if (strip && use_s2_tb(h)) {
-    a.s2_tb = 1;
-    a.s2_lo = a.strip_a + 2;
-    a.s2_hi = a.strip_b - 2;
-  }
+  if (strip) set_s2(h, a);
   a.phase = PH_B; a.s_in = SP1; a.s_out = SP2;
   if ((e = enqueue_phase(h, a, pass, false, strip)) != hipSuccess) return e;
   // corrector tendency T = L(S2) and the beta inner-product partials
@@ -1625,7 +1634,7 @@ int gd_time_kernel(gd_handle *h, int32_t kernel, int32_t reps, double *us) {
   if (kernel == GD_TIME_FILTER && h->frows.empty()) return fail(h, GD_ERR_INVALID_ARG, "no filtered rows");
   if (kernel == GD_TIME_FILTER_MM && (!h->filt_mm || h->mslots.empty()))
     return fail(h, GD_ERR_NOT_SUPPORTED, "the handle does not filter on the matrix cores");
-  if (kernel == GD_TIME_PHASE && !use_fused(h))
+  if (kernel == GD_TIME_PHASE && step_form(h) == 0)
     return fail(h, GD_ERR_NOT_SUPPORTED, "the handle does not use fused phase launches");
   hipSetDevice(h->device);
   // arguments of the second predictor of a fast-pass call (predict_correct,
@@ -1651,7 +1660,11 @@ int gd_time_kernel(gd_handle *h, int32_t kernel, int32_t reps, double *us) {
   GD_HIP(h, hipEventCreate(&e0));
   GD_HIP(h, hipEventCreate(&e1));
   auto one = [&]() -> hipError_t {
-    if (kernel == GD_TIME_TEND) return launch_tend(a, h->prec, pass, false, h->stream);
+    if (kernel == GD_TIME_TEND) {
+      Args f = a;
+      if (set_strips(h, f, pass, h->nmem)) set_ranges(f, h->near_all, h->nmem);
+      return launch_tend(f, h->prec, pass, false, h->stream);
+    }
     if (kernel == GD_TIME_FILTER) {
       Args f = a;
       f.ntiles = (int)h->frows.size();
@@ -1660,7 +1673,8 @@ int gd_time_kernel(gd_handle *h, int32_t kernel, int32_t reps, double *us) {
     if (kernel == GD_TIME_PHASE) {
       Args f = a;
       const bool strip = set_strips(h, f, pass, h->nmem);
-      const int form = strip ? strip_form(h) : phase_form(h);
+      const int form = step_form(h);
+      if (strip) set_s2(h, f);
       set_fused(h, f, h->nmem, strip ? h->near_far : h->far);
       if (form == 3) return launch_rphase(f, h->prec, pass, false, h->stream);
       if (form == 2) return launch_wphase(f, h->prec, pass, false, h->stream);

@@ -398,36 +398,42 @@ int64_t gd_device_bytes(const gd_handle *h);
  * state X is not modified).  kernel: GD_TIME_TEND (tendency kernel, fast
  * pass, second predictor), GD_TIME_FILTER (the filter of that phase),
  * GD_TIME_UPDATE (beta + corrector), GD_TIME_PHASE (that phase as one fused
- * launch, in the form and with the strip tiles the step gives it, storing its
- * predictor in full: tendency, filter rows and epilogue; GD_ERR_NOT_SUPPORTED when the handle steps with separate
- * tendency and filter launches), GD_TIME_FILTER_MM
- * (the matrix-core projection of the momentum rows of every member; the
- * mixed_mfma and mixed_bf16 modes only).  No counterpart in the reference: a
- * measurement hook. */
+ * launch: tendency, filter rows and epilogue; GD_ERR_NOT_SUPPORTED when the
+ * handle's steps make separate tendency and filter launches),
+ * GD_TIME_FILTER_MM (the matrix-core projection of the momentum rows of every
+ * member; the mixed_mfma and mixed_bf16 modes only).  The tendency and phase
+ * launches have the form, the strip tiles and the predictor store that a
+ * step gives them.  No counterpart in the reference: a measurement hook. */
 enum { GD_TIME_TEND = 0, GD_TIME_FILTER = 1, GD_TIME_UPDATE = 2, GD_TIME_PHASE = 3, GD_TIME_FILTER_MM = 4 };
 
-/* How the handle's step, at its current active-member count, launches each
- * tendency phase: 0 a tendency launch then a filter launch, 1 one fused
- * launch (tendency, filter rows and epilogue), 2 one fused launch in
+/* Form of the handle's tendency phase launches without strip tiles, at its
+ * current active-member count: 0 a tendency launch then a filter launch, 1 one
+ * fused launch (tendency, filter rows and epilogue), 2 one fused launch in
  * workgroups of two row segments (a filtered row's segments evaluated two at
- * a time; rows of 255 to 762 longitudes).  By default phases are fused with
- * filtered rows while active members x num_lat x ceil(num_lon/254) row
- * tiles stay within 24576 (num_lon <= 1024) or 6144 (num_lon <= 2048), in
- * form 2 for rows of 255 to 508 longitudes while its workgroups (filtered
- * rows plus far rows) fit two per compute unit; gd_autotune may choose any
- * form.  In the calls of csp2 the rows away from the polar filter run as strip
- * tiles (several rows each) beside the launch's other rows, and the form is
- * then chosen by its filtered rows: 2, 1, or one fused launch with a workgroup
- * per filtered row (num_lon <= 1024).  This function reports the form of the
- * other launches (a forced or tuned 3 as 1); gd_profile_kernels names the
- * launches of a step (phase, wphase, rphase).
- * GD_FUSED=0, 1, 2 or 3 in the environment when the handle is created forces
- * a form (2 falls back to 1 outside 255 to 762 longitudes; 3, the workgroup
- * per filtered row, to 1 where a launch cannot take it); GD_STRIP=n gives the
- * rows per strip tile (0: none), GD_FOLD=0 or 1 whether such calls leave their
- * update to the next call's first launch (by grid size when absent), GD_S2TB=0 or
- * 1 whether their strip tiles form the second predictor again in the corrector
- * phase instead of loading it (by batch size when absent).  Every form gives the same bits.  No
+ * a time; rows of 255 to 762 longitudes).  These are the launches of unsplit
+ * and isp steps and of gd_space_operators, and the last diffusion application
+ * is fused where this is not 0.  By default phases are fused with filtered
+ * rows while active members x num_lat x ceil(num_lon/254) row tiles stay
+ * within 24576 (num_lon <= 1024) or 6144 (num_lon <= 2048), in form 2 for rows
+ * of 255 to 508 longitudes while its workgroups (filtered rows plus far rows)
+ * fit two per compute unit; gd_autotune may choose any form.
+ *
+ * In the calls of csp2 the rows away from the polar filter run as strip tiles
+ * (several rows each) beside the launch's other rows.  Such a launch is fused
+ * at any size where it can be (filtered rows, num_lon <= 2048), in form 2, 1,
+ * or 3: one fused launch with a workgroup per filtered row (num_lon <= 1024).
+ * This function does not report them (a forced or tuned 3 counts as 1);
+ * gd_profile_kernels names the launches of a step: tend and filter, phase,
+ * wphase, rphase, and phase_s2tb or rphase_s2tb for a corrector phase whose
+ * strip tiles form the second predictor again.
+ *
+ * In the environment when the handle is created: GD_FUSED=0, 1, 2 or 3 forces
+ * a form (2 falls back to 1 outside 255 to 762 longitudes; 3 to 1 where a
+ * launch cannot take it); GD_STRIP=n gives the rows per strip tile (0: none);
+ * GD_FOLD=0 or 1 whether csp2's calls leave their update to the next call's
+ * first launch (by grid size when absent); GD_S2TB=0 or 1 whether strip tiles
+ * form the second predictor again in the corrector phase instead of loading it
+ * (by batch size when absent).  Every form gives the same bits.  No
  * counterpart in the reference. */
 int gd_fused_phases(const gd_handle *h);
 
