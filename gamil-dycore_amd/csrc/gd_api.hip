@@ -300,10 +300,11 @@ void set_fused(const gd_handle *h, Args &a, int nm, const RowRanges &r) {
   set_ranges(a, r, nm);
 }
 
-// Fused phase launches pay off while a launch is a few rounds of resident
-// tiles (latency bound); past that the lower occupancy of k_phase (five
-// tiles per CU against seven or eight for k_tend) costs more than the
-// launches it saves.  Measured on MI355X (mixed, aggregate model-days/s):
+// Fused phase launches without strip tiles pay off while a launch is a few
+// rounds of resident tiles (latency bound); past that the lower occupancy of
+// k_phase (five tiles per CU against seven or eight for k_tend) costs more than
+// the launches it saves.  (With strip tiles they pay at any size: strip_form.)
+// Measured on MI355X (mixed, aggregate model-days/s):
 // fused still ahead at 16 runs of 720x361 (17,328 tiles), 64 members of
 // 360x181 (23,168) and 128 of 180x91 (11,648); even at 32 runs of 720x361
 // (34,656).
@@ -313,7 +314,8 @@ constexpr int64_t kFusedMaxTiles = 24576;
 // larger launches are left to the autotuner.
 constexpr int64_t kFusedMaxTilesWide = 6144;
 
-// Form of the phase launches: 0 k_tend + k_filter, 1 k_phase, 2 k_wphase.
+// Form of the phase launches without strip tiles: 0 k_tend + k_filter, 1
+// k_phase, 2 k_wphase.
 // k_wphase for rows of two segments by default while its workgroups -- one
 // per filter row and one per far row -- fit two per CU: measured on MI355X
 // (mixed, one or two runs of 288x145, 360x181, 480x241) 3-10% faster than
@@ -353,6 +355,14 @@ bool has_strips(const gd_handle *h) { return h->strip_b >= h->strip_a && strip_r
 
 // Form of the phase launches of a call with strip tiles, unless the handle's
 // form is forced or tuned: 1 k_phase, 2 k_wphase, 3 k_rphase.
+// Separate launches (0) only where nothing can be fused: they lose at every size
+// measured, also past phase_form's limits.  ms per step separate / k_phase / k_rphase: 64
+// of 360x181 (23,168 row tiles) 3.98 / 3.75 / 3.29, 96 (34,752) 5.86 / 5.62 /
+// 4.96, 160 (57,920) 9.47 / 9.29 / 8.22, 32 of 720x361 (34,656) 6.20 / 5.86 /
+// 5.65, 320 of 180x91 (29,120) 5.73 / 5.45 / 4.40, 16 of 1024x513 (41,040) 6.63
+// / 6.17 / 6.96; past 1024 longitudes separate / k_phase: 2, 4, 8 of 1440x721
+// (8,652 to 34,608) 1.73 / 1.43, 3.41 / 3.03, 6.42 / 5.95, 2 of 2048x1025
+// (18,450) 3.83 / 3.24.
 // k_wphase (shortest chain of a filter row) while its workgroups fit about two
 // per CU: 360x181 0.241 ms per step against 0.267 (k_phase) and 0.327
 // (k_rphase), four of them 0.326 / 0.341 / 0.395, 720x361 0.355 / 0.366 /
@@ -424,11 +434,12 @@ struct Pending {
   double dt = 0;
 };
 
-// Whether csp2's calls leave their update to the next call's phase A (GD_FOLD
-// = 0 or 1 in the environment when the handle is created overrides), which then takes the call's Tc beside its state and adds the beta partials in
-// every tile: one launch and its gap less per call, against num_lat * segments
-// more entries of 48 bytes to read per tile.  ms per step with the k_update
-// launches and without: 180x90 0.256 / 0.243, 8 members of 180x91 0.279 / 0.249,
+// Whether csp2's calls leave their update to the next call's phase A (GD_FOLD =
+// 0 or 1 in the environment when the handle is created overrides), which then
+// takes the call's Tc beside its state and adds the beta partials in every
+// tile: one launch and its gap less per call, against num_lat * segments more
+// entries of 48 bytes to read per tile.  ms per step with the k_update launches
+// and without: 180x90 0.256 / 0.243, 8 members of 180x91 0.279 / 0.249,
 // 360x181 0.240 / 0.227, 405x203 0.350 / 0.336, 720x361 (1083 entries) 0.355 /
 // 0.350, two of them 0.464 / 0.442; 900x451 (1804 entries) 0.541 / 0.550,
 // 1440x721 (4326) 0.730 / 0.747.  A launch of many rounds hides the k_update
@@ -448,10 +459,11 @@ bool use_fold(const gd_handle *h) {
 // read it, so that phase B stores S2 only next to other tiles (GD_S2TB = 0 or
 // 1 in the environment when the handle is created overrides): three field
 // stores fewer per call, for loads of two fields in place of one in phase C.
-// It pays where a call's fields (three each of S0, S1, S2, Tb, Tc, and ghs) no
-// longer stay in the 256 MB memory-side cache.  ms per step without and with:
-// 24 of 360x181 (214 MB) 1.168 / 1.088, 64 of them (570 MB) 3.328 / 3.277, 6 of
-// 720x361 (204 MB) 1.036 / 1.004, 8 of them (272 MB) 1.417 / 1.349, 128 of
+// It pays from somewhere between 142 and 204 MB of a call's fields (three each
+// of S0, S1, S2, Tb, Tc, and ghs) on, where they begin to leave the 256 MB
+// memory-side cache, which a launch's other data share.  ms per step without
+// and with: 24 of 360x181 (214 MB) 1.168 / 1.088, 64 of them (570 MB) 3.328 /
+// 3.277, 6 of 720x361 (204 MB) 1.036 / 1.004, 8 of them (272 MB) 1.417 / 1.349, 128 of
 // 180x91 (286 MB) 1.727 / 1.633, 2 of 1440x721 (266 MB) 1.510 / 1.433; below,
 // the loads cost more than the stores: 16 of 360x181 (142 MB) 0.758 / 0.768, 4 of
 // 720x361 (136 MB) 0.706 / 0.721, one 1440x721 (133 MB) 0.730 / 0.760.

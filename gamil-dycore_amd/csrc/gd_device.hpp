@@ -122,11 +122,11 @@ struct Args {
   int mm;                      // k_filter: momentum rows come projected in sy (MFMA modes)
   const double *twid;          // [N/2+1][2]: cos, sin of 2 pi k / N
   const double *ghost;         // [2][pitch]: a row of 1.0 and a row of 0.0, read for rows beyond the grid
-  // k_filter projection (PH_P): rows at sx_ext + slot * pitch, or with sx_ld
-  // (then not 0) in place at sx_ext + row * sx_ld
+  // k_filter projection (PH_P): rows at sx_ext + slot * pitch instead of the
+  // member's staging rows (nullptr: the member's), or with sx_ld (not 0) in
+  // place at sx_ext + row * sx_ld
   double *sx_ext;
   int64_t sx_ld;
-                               // instead of the member's staging rows (nullptr: the member's)
   int fft_L;                   // complex FFT length: N/2 (even N) or N
   int fft_half;                // 1: even N, real FFT through a half-length complex FFT
   int fft_nrad;                // radix passes

@@ -67,7 +67,11 @@ __device__ __forceinline__ StripRow<CT> strip_row(const Args &a, int row) {
   return b;
 }
 
-// x / d with r = 1/d rounded to nearest.
+// x / d with r = 1/d rounded to nearest: Markstein's division by a divisor known
+// in advance, one product and two fused steps, which rounds as the division does
+// where nothing over- or underflows (Brisebarre, Muller and Raina, IEEE
+// Transactions on Computers 53(8), 2004); the fixup gives zeros, infinities and
+// NaN the division's result.
 __device__ __forceinline__ double divu(double x, double d, double r) {
   double q = x * r;
   q = __builtin_fma(__builtin_fma(-q, d, x), r, q);

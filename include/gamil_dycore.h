@@ -13,7 +13,9 @@
  * Conventions
  *   - Return value: GD_OK (0) or a GD_ERR_* code; gd_last_error() gives text.
  *   - The caller owns host buffers, the library owns device buffers; no host
- *     pointer is kept after a call returns.
+ *     pointer is kept after a call returns.  Field copies go through pinned host
+ *     memory that a handle keeps until gd_destroy (its largest copy so far, at
+ *     most 32 MiB).
  *   - Host field layout: pointer to element (i=1, j=1), longitude fastest,
  *     consecutive latitude rows `ld` elements apart (ld >= num_lon).  A
  *     Fortran halo'd array x(-1:N+2,-1:M+2) is passed as x(1,1) with
